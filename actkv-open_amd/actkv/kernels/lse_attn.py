@@ -2,7 +2,7 @@
 
 Drop-in for the reference module actkv/kernels/lse_attn.py: same names, arguments, in-place
 semantics and errors.  `action_scores` runs the HIP kernels of libactkv_hip.so (bf16/fp16
-MFMA kernels for head_dim 128 or 64 and 1 to 16 query heads per KV head; a VALU kernel for
+MFMA kernels for head_dim 256, 128 or 64 and 1 to 16 query heads per KV head; a VALU kernel for
 every other shape and for float32 caches).  It has no CPU path: CPU tensors raise.
 
 Layout (vLLM-style), one layer:

@@ -10,8 +10,8 @@
 // out and lse are float32.  A row that sees no token gets lse = -inf, out = 0
 // (torch's logsumexp and softmax-einsum over an empty set).
 //
-// MFMA path (bf16/fp16, head_dim 128 or 64, any GQA group, more than one 32-row tile
-// of query rows per pair): FlashAttention-style,
+// MFMA path (bf16/fp16, head_dim 256, 128 or 64, any GQA group, more than one 32-row tile
+// of query rows per pair; any number at head dim 256): FlashAttention-style,
 // one workgroup per (layer, request, KV head, group of NW row tiles), NW waves,
 // each owning one 32-row tile of the pair's query rows (n, g) and streaming all
 // of the request's tokens.  The transposed products keep every per-query
@@ -29,7 +29,7 @@
 // bit, several stages ahead), rows XOR-swizzled; V is read back transposed
 // (ds_read_b64_tr_b16).  Described at attn_ring_kernel.
 //
-// Decode path (the same dtypes and shapes when a pair's query rows fit one 32-row
+// Decode path (head dims 128 and 64, the same dtypes, when a pair's query rows fit one 32-row
 // tile, N*G <= 32): four waves per (pair, token chunk), each streaming its own
 // slices through a private LDS region without workgroup barriers; V comes back
 // transposed from LDS (ds_read_b64_tr_b16).  Described at attn_decode_kernel.
@@ -37,6 +37,13 @@
 // Head dim 64 runs the same kernels with half-length token rows: a 16-byte load
 // instruction then moves eight rows instead of four, the rows' eight 16-byte chunks are
 // swizzled with their own pattern (dswz), and two 32-dim output tiles replace four.
+//
+// Head dim 256 runs the ring kernel for every row count, one wave per SIMD (a wave's O tile is 128
+// registers, its query rows 64), with P as three terms in bf16.  16 query heads over 8 KV heads
+// in bf16, against the float32 path these shapes took before: 24 causal queries over 12000 and
+// 5003 tokens, attention and scoring together, 742 -> 102 us; a decode step over 8 x 8k tokens
+// 310 -> 182 us; 700 causal queries over 3000 and 2003 tokens 2555 -> 266 us.  out is 5.5e-7 to
+// 6.9e-7 from 64 bits on them, against 7.7e-7 to 9.1e-7.
 //
 // Generic path (any other dtype / head_dim up to 512 / block size): float32, up to 8
 // query rows of one KV head per workgroup (a decode step's GQA group of up to 8 heads
@@ -106,23 +113,25 @@ __device__ __forceinline__ int attn_phys(const AttnArgs &a, int r, int b) {
 template <int DH>
 __device__ __forceinline__ void attn_merge_row(const AttnArgs &a, int64_t id, int nc, int64_t o_off,
                                                int64_t lse_off, int lane) {
-  static_assert(DH == 64 || DH == 128, "head dims");
-  constexpr int PRE = 16;
+  static_assert(DH == 64 || DH == 128 || DH == 256, "head dims");
+  constexpr int PRE = 16, DL = DH / 64;
   const float *ml = a.ws_ml + id * a.nchunk * 2;
   const float *wo = a.ws_o + id * a.nchunk * DH;
-  float pre0[PRE], pre1[PRE];
+  float pre[DL][PRE];
 #pragma unroll
   for (int j = 0; j < PRE; ++j) {
     const int jc = max(0, min(j, nc - 1));  // an in-bounds row: the workspace holds nchunk >= max(nc, 1)
-    pre0[j] = wo[(int64_t)jc * DH + lane];
-    if constexpr (DH == 128) pre1[j] = wo[(int64_t)jc * DH + 64 + lane];
+#pragma unroll
+    for (int k = 0; k < DL; ++k) pre[k][j] = wo[(int64_t)jc * DH + 64 * k + lane];
   }
   float M = -INFINITY;
   for (int c = lane; c < nc; c += 64) M = fmaxf(M, ml[2 * c]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
   const float Ms = M == -INFINITY ? 0.f : M;
-  float Lsum = 0.f, o0 = 0.f, o1 = 0.f;
+  float Lsum = 0.f, ov[DL];
+#pragma unroll
+  for (int k = 0; k < DL; ++k) ov[k] = 0.f;
   for (int c0 = 0; c0 < nc; c0 += 64) {
     const int c = c0 + lane;
     const float w = c < nc ? __builtin_amdgcn_exp2f(ml[2 * c] - Ms) : 0.f;
@@ -134,21 +143,21 @@ __device__ __forceinline__ void attn_merge_row(const AttnArgs &a, int64_t id, in
 #pragma unroll
       for (int j = 0; j < PRE; ++j) {
         const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
-        o0 += j < nc ? wj * pre0[j] : 0.f;
-        if constexpr (DH == 128) o1 += j < nc ? wj * pre1[j] : 0.f;
+#pragma unroll
+        for (int k = 0; k < DL; ++k) ov[k] += j < nc ? wj * pre[k][j] : 0.f;
       }
     }
     const float *wc = wo + (int64_t)c0 * DH;
     for (int j = c0 == 0 ? PRE : 0; j < min(64, nc - c0); ++j) {
       const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
-      o0 += wj * wc[j * DH + lane];
-      if constexpr (DH == 128) o1 += wj * wc[j * DH + 64 + lane];
+#pragma unroll
+      for (int k = 0; k < DL; ++k) ov[k] += wj * wc[j * DH + 64 * k + lane];
     }
   }
   const float inv = Lsum > 0.f ? 1.0f / Lsum : 0.f;
   float *op = a.out + o_off;
-  op[lane] = o0 * inv;
-  if constexpr (DH == 128) op[64 + lane] = o1 * inv;
+#pragma unroll
+  for (int k = 0; k < DL; ++k) op[64 * k + lane] = ov[k] * inv;
   if (lane == 0) a.lse[lse_off] = Lsum > 0.f ? (M + __log2f(Lsum)) * 0.6931471805599453f : -INFINITY;
 }
 
@@ -204,8 +213,8 @@ constexpr int DW = 4;                         // waves per decode workgroup
 // bytes, NC 16-byte chunks (NC = 2^NCS); a 64-lane 16-byte load moves RPI = 2^RPS rows;
 // the S^T product takes KS 16-dim steps and O^T has DT 32-dim tiles.
 template <int DH> struct RowShape {
-  static_assert(DH == 64 || DH == 128, "head dims");
-  static constexpr int PB = 2 * DH, NC = PB / 16, NCS = NC == 16 ? 4 : 3;
+  static_assert(DH == 64 || DH == 128 || DH == 256, "head dims");
+  static constexpr int PB = 2 * DH, NC = PB / 16, NCS = NC == 32 ? 5 : NC == 16 ? 4 : 3;
   static constexpr int RPI = 64 / NC, RPS = 6 - NCS;
   static constexpr int KS = DH / 16, DT = DH / 32;
   static constexpr int DREG = 2 * 32 * PB;    // decode LDS bytes per wave: K rows, then V rows
@@ -224,7 +233,7 @@ __device__ __forceinline__ int attn_dec_chunks(const AttnArgs &a, int S) {
 // address's 16-byte unit mod 16), so no LDS bank conflicts, for: 16 consecutive tokens at
 // one chunk (K A-operand reads); four consecutive tokens at four consecutive chunks (a
 // 32-lane transposed V read: 16 slots); the chunks of one row (row writes).
-//   Head dim 128 (16 chunks, a row is 16 units): 4 (t mod 4) + (t / 4 mod 4).  2 (t mod 8)
+//   Head dim 128 (16 chunks, a row is 16 units; head dim 256, 32 chunks, the same modulo 16): 4 (t mod 4) + (t / 4 mod 4).  2 (t mod 8)
 //   + (t / 8 mod 2) left the transposed V reads 2-way conflicted.
 //   Head dim 64 (8 chunks, a row is 8 units, so rows of odd t use units 8-15): 4 (t / 2 mod 2)
 //   + (t / 4 mod 4).  Among 16 tokens each parity takes all 8 values; tokens 4m and 4m + 2
@@ -232,7 +241,7 @@ __device__ __forceinline__ int attn_dec_chunks(const AttnArgs &a, int S) {
 //   disjoint halves.
 template <int DH>
 __device__ __forceinline__ int dswz(int t) {
-  if constexpr (DH == 128) return 4 * (t & 3) + ((t >> 2) & 3);
+  if constexpr (DH >= 128) return 4 * (t & 3) + ((t >> 2) & 3);
   else return 4 * ((t >> 1) & 1) + ((t >> 2) & 3);
 }
 
@@ -527,9 +536,13 @@ __device__ __forceinline__ void lds_barrier() {
 // 4 requests x 8k tokens x 48 causal queries: with the loads issued ahead, depth matters
 // little (3 or 4 stages of 64 tokens and 2 of 128 are within 8%) and fewer, larger stages
 // (fewer barriers) win; 4- and 2-wave workgroups keep 64-token stages so that two fit
-// per CU.
+// per CU.  Head dim 256: what fits twice per CU (32 tokens of K and V are 32 KB) for one and two
+// waves, 64 tokens for four.
+constexpr int ring_stage(int tiles, int dh) {
+  return dh == 256 ? (tiles >= 4 ? 64 : 32) : tiles >= 8 ? 128 : 64;
+}
 template <int TILES, int DH> struct RingShape {             // TILES: row tiles per workgroup
-  static constexpr int ST = TILES >= 8 ? 128 : 64;            // tokens per stage
+  static constexpr int ST = ring_stage(TILES, DH);            // tokens per stage
   static constexpr int NSTG = 2;                              // ring depth
   static constexpr int TBLW = TILES >= 8 ? 4096 : 2048;       // block-table window (entries)
   static constexpr int SBYTES = 2 * ST * RowShape<DH>::PB;    // K then V rows of a stage
@@ -562,7 +575,7 @@ __device__ __forceinline__ void buf_lds16(ri32x4 rsrc, unsigned voff, unsigned l
 
 template <typename T, typename V8, int DH, int NW, int RT, bool CAUSAL>
 __global__ void __launch_bounds__(NW * 64)
-__attribute__((amdgpu_waves_per_eu(RT >= 2 ? 1 : (NW >= 4 ? 2 : 1), RT >= 2 ? 1 : 2)))
+__attribute__((amdgpu_waves_per_eu(RT >= 2 || DH == 256 ? 1 : (NW >= 4 ? 2 : 1), RT >= 2 || DH == 256 ? 1 : 2)))
 attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
   const int G = a.G;   // query heads per KV head: rows (n, g) of a tile are independent
   using SH = RingShape<NW * RT, DH>;
@@ -570,6 +583,10 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
   constexpr int PB = RS::PB, NC = RS::NC, NCS = RS::NCS, RPI = RS::RPI, KS = RS::KS, DT = RS::DT;
   constexpr int ST = SH::ST, NSTG = SH::NSTG, TBLW = SH::TBLW;
   constexpr int PER = 2 * SH::IPP / NW;  // load instructions per wave per stage
+  // bf16 at head dim 256: a third term gives P 24 significant bits, as many as the float32 path
+  // that serves the other dtypes there (with hi + lo alone out was 1.3e-6 from 64 bits on
+  // causal prefill against that path's 7.7e-7)
+  constexpr bool P3 = DH == 256 && __is_same(T, __bf16);
   static_assert((2 * SH::IPP) % NW == 0, "whole load instructions per wave");
   __shared__ __attribute__((aligned(1024))) unsigned char ring[NSTG][SH::SBYTES];
   __shared__ int tbl[TBLW];
@@ -727,7 +744,7 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
   // online softmax of each tile's rows over the slice, then O^T += V^T . P^T with each V^T
   // fragment read once for all tiles
   auto softmax_pv = [&](Tiles &st, const unsigned char *vl, int t0) {
-    V8 pb[RT][2], pbl[RT][2];  // P = hi + lo, both in the cache dtype
+    V8 pb[RT][2], pbl[RT][2], pbm[RT][2];  // P = hi + lo (+ a third term), in the cache dtype
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       f32x16 &x = st.s[rt];
@@ -755,7 +772,10 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
         ps += pe;
         const T hi = (T)pe;
         pb[rt][e >> 3][e & 7] = hi;
-        pbl[rt][e >> 3][e & 7] = (T)(pe - (float)hi);
+        const float res = pe - (float)hi;
+        const T lo = (T)res;
+        pbl[rt][e >> 3][e & 7] = lo;
+        if constexpr (P3) pbm[rt][e >> 3][e & 7] = (T)(res - (float)lo);
       }
       {
         const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(ps), __float_as_uint(ps), false, false);
@@ -789,6 +809,8 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
           if constexpr (__is_same(T, __bf16)) {
             oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pb[rt][kb], oacc[rt][dt], 0, 0, 0);
             oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pbl[rt][kb], oacc[rt][dt], 0, 0, 0);
+            if constexpr (P3)
+              oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pbm[rt][kb], oacc[rt][dt], 0, 0, 0);
           } else {
             oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pb[rt][kb], oacc[rt][dt], 0, 0, 0);
             oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pbl[rt][kb], oacc[rt][dt], 0, 0, 0);
@@ -1102,9 +1124,10 @@ __global__ void __launch_bounds__(256) attn_generic_kernel(AttnArgs a, int pairs
 // one tile per wave at two waves per SIMD (36 layers x 32k x 128 queries): the second
 // wave hides more than the halved LDS reads save.
 struct RingCfg { int nw, rt; };
-static RingCfg ring_cfg(int rtiles) {
+static RingCfg ring_cfg(int rtiles, int D) {
+  if (rtiles == 1) return {1, 1};   // head dim 256 only
   if (rtiles <= 2) return {2, 1};
-  if (rtiles <= 4) return {4, 1};
+  if (rtiles <= 4 || D == 256) return {4, 1};
   return {8, 1};
 }
 
@@ -1125,10 +1148,10 @@ static int device_cus() {
   return cached[dev];
 }
 
-static AttnSplit attn_split(int pairs, int N, int G, int span, int cus) {
+static AttnSplit attn_split(int pairs, int N, int G, int D, int span, int cus) {
   AttnSplit sp;
   const int rtiles = (N * G + 31) / 32;
-  if (rtiles == 1) {
+  if (rtiles == 1 && D != 256) {
     // decode kernel: DW waves per (pair, chunk), two resident workgroups per CU.  With few
     // pairs the chunks stop at about 1.5 workgroups per CU, within one round: a served decode
     // step's per-layer call (32 pairs x 4400 tokens) took 27.7 / 28.1 / 26.1 / 28.3 / 31.7 /
@@ -1146,12 +1169,12 @@ static AttnSplit attn_split(int pairs, int N, int G, int span, int cus) {
     sp.tpc = sp.nchunk > 1 ? 0 : std::max(span, 1);
     return sp;
   }
-  const RingCfg cfg = ring_cfg(rtiles);
+  const RingCfg cfg = ring_cfg(rtiles, D);
   const int tiles = cfg.nw * cfg.rt;
-  const int st = tiles >= 8 ? 128 : 64;  // ring stage (RingShape<tiles>::ST)
+  const int st = ring_stage(tiles, D);
   sp.ngroups = (rtiles + tiles - 1) / tiles;
-  sp.rows_pad = sp.ngroups * tiles * 32;
-  const int per_cu = tiles >= 8 ? 1 : 2;  // resident ring workgroups per CU (LDS)
+  sp.rows_pad = N * G;   // only rows that exist are written and merged
+  const int per_cu = tiles >= 8 || D == 256 ? 1 : 2;  // resident ring workgroups per CU (LDS)
   const int64_t items = (int64_t)pairs * sp.ngroups;
   const int64_t want = 4LL * 256 * per_cu;
   int nchunk = (int)std::min<int64_t>(std::max<int64_t>(1, (want + items - 1) / items), std::max(1, span / 256));
@@ -1173,22 +1196,25 @@ static int launch_attn_mfma(AttnArgs a, int bs_shift, void *ws, size_t ws_bytes,
   const int pairs = a.L * a.R * a.Hkv;
   const int rtiles = (a.N * a.G + 31) / 32;
   const bool causal = a.kv_len != nullptr;
-  AttnSplit sp = attn_split(pairs, a.N, a.G, a.max_blocks * a.BS, device_cus());
+  AttnSplit sp = attn_split(pairs, a.N, a.G, DH, a.max_blocks * a.BS, device_cus());
   const size_t need = attn_ws_bytes(pairs, sp, DH);
   if (sp.nchunk > 1 && (!ws || ws_bytes < need)) {  // no (large enough) workspace: no split
     sp.nchunk = 1;
     sp.tpc = std::max(a.max_blocks * a.BS, 1);
   }
   a.nchunk = sp.nchunk; a.tpc = sp.tpc; a.rows_pad = sp.rows_pad;
-  a.dyn = rtiles == 1 && sp.nchunk > 1;
+  const bool decode = rtiles == 1 && DH != 256;
+  a.dyn = decode && sp.nchunk > 1;
   a.ws_o = sp.nchunk > 1 ? (float *)ws : nullptr;
   a.ws_ml = sp.nchunk > 1 ? (float *)((char *)ws + (size_t)pairs * sp.rows_pad * sp.nchunk * DH * sizeof(float)) : nullptr;
-  if (rtiles == 1) {
-    const int grid = pairs * sp.nchunk;
-    if (causal)
-      hipLaunchKernelGGL((attn_decode_kernel<T, V8, DH, true>), dim3(grid), dim3(DW * 64), 0, st, a, pairs, bs_shift);
-    else
-      hipLaunchKernelGGL((attn_decode_kernel<T, V8, DH, false>), dim3(grid), dim3(DW * 64), 0, st, a, pairs, bs_shift);
+  if (decode) {
+    if constexpr (DH != 256) {
+      const int grid = pairs * sp.nchunk;
+      if (causal)
+        hipLaunchKernelGGL((attn_decode_kernel<T, V8, DH, true>), dim3(grid), dim3(DW * 64), 0, st, a, pairs, bs_shift);
+      else
+        hipLaunchKernelGGL((attn_decode_kernel<T, V8, DH, false>), dim3(grid), dim3(DW * 64), 0, st, a, pairs, bs_shift);
+    }
   } else {
 #define ACTKV_ATTN(NWV, RTV)                                                                       \
   do {                                                                                             \
@@ -1200,10 +1226,16 @@ static int launch_attn_mfma(AttnArgs a, int bs_shift, void *ws, size_t ws_bytes,
       hipLaunchKernelGGL((attn_ring_kernel<T, V8, DH, NWV, RTV, false>), dim3(grid), dim3(NWV * 64),\
                          0, st, a, pairs, sp.ngroups, bs_shift);                                   \
   } while (0)
-  const RingCfg cfg = ring_cfg(rtiles);
-  if (cfg.nw == 2) ACTKV_ATTN(2, 1);
-  else if (cfg.nw == 4) ACTKV_ATTN(4, 1);
-  else ACTKV_ATTN(8, 1);
+  const RingCfg cfg = ring_cfg(rtiles, DH);
+  if (cfg.nw == 2) {
+    ACTKV_ATTN(2, 1);
+  } else if constexpr (DH == 256) {
+    if (cfg.nw == 1) ACTKV_ATTN(1, 1);
+    else ACTKV_ATTN(4, 1);
+  } else {
+    if (cfg.nw == 4) ACTKV_ATTN(4, 1);
+    else ACTKV_ATTN(8, 1);
+  }
 #undef ACTKV_ATTN
   }
   int rc = actkv_check_launch();
@@ -1327,15 +1359,17 @@ extern "C" int actkv_paged_attention(
                       kv_sl % 8 == 0 && kv_sv % 8 == 0 && kv_sb % 8 == 0 && kv_ss % 8 == 0 &&
                       kv_sh % 8 == 0 && o_sl % 4 == 0 && o_sr % 4 == 0 && o_sn % 4 == 0 && o_sh % 4 == 0;
   const bool mfma_ok = q_dtype == kv_dtype && (kv_dtype == ACTKV_BF16 || kv_dtype == ACTKV_F16) &&
-                       (D == 128 || D == 64) && G >= 1 && vec_ok && bs_shift >= 0;
+                       (D == 256 || D == 128 || D == 64) && G >= 1 && vec_ok && bs_shift >= 0;
   if (mfma_ok) {
     void *ws = workspace;
     const size_t wb = workspace_bytes;
     if (kv_dtype == ACTKV_BF16)
-      return D == 64 ? launch_attn_mfma<__bf16, bf16x8, 64>(a, bs_shift, ws, wb, st)
-                     : launch_attn_mfma<__bf16, bf16x8, 128>(a, bs_shift, ws, wb, st);
-    return D == 64 ? launch_attn_mfma<_Float16, f16x8, 64>(a, bs_shift, ws, wb, st)
-                   : launch_attn_mfma<_Float16, f16x8, 128>(a, bs_shift, ws, wb, st);
+      return D == 64    ? launch_attn_mfma<__bf16, bf16x8, 64>(a, bs_shift, ws, wb, st)
+             : D == 128 ? launch_attn_mfma<__bf16, bf16x8, 128>(a, bs_shift, ws, wb, st)
+                        : launch_attn_mfma<__bf16, bf16x8, 256>(a, bs_shift, ws, wb, st);
+    return D == 64    ? launch_attn_mfma<_Float16, f16x8, 64>(a, bs_shift, ws, wb, st)
+           : D == 128 ? launch_attn_mfma<_Float16, f16x8, 128>(a, bs_shift, ws, wb, st)
+                      : launch_attn_mfma<_Float16, f16x8, 256>(a, bs_shift, ws, wb, st);
   }
   switch (q_dtype) {
     case ACTKV_F32: return dispatch_attn_generic<float>(a, kv_dtype, workspace, workspace_bytes, st);
@@ -1351,8 +1385,9 @@ extern "C" size_t actkv_paged_attention_workspace_size(int L, int R, int N, int 
   if (G < 1 || D > 512) return 0;
   if ((int64_t)max_blocks * block_size > 0x7fffffffLL) return 0;
   const int pairs = L * R * Hkv;
-  // head dims 128 and 64: the matrix-core split; others: the float32 path's split
-  if (D == 128 || D == 64)
-    return attn_ws_bytes(pairs, attn_split(pairs, N, G, max_blocks * block_size, device_cus()), D);
-  return attn_ws_bytes(pairs, attn_split_generic(pairs, N, G, max_blocks * block_size, device_cus()), D);
+  // head dims 256, 128 and 64 take the matrix-core split or, with a dtype or block size off that
+  // path, the float32 path's: room for either
+  const size_t gen = attn_ws_bytes(pairs, attn_split_generic(pairs, N, G, max_blocks * block_size, device_cus()), D);
+  if (D != 256 && D != 128 && D != 64) return gen;
+  return std::max(gen, attn_ws_bytes(pairs, attn_split(pairs, N, G, D, max_blocks * block_size, device_cus()), D));
 }

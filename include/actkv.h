@@ -75,10 +75,10 @@ const char *actkv_version(void);
  * out   : float32 [L, R, Hkv, W], strides out_sl out_sr out_sh, unit last,
  *         W >= max_blocks*block_size (checked)
  * scale : softmax scale (the reference default is head_dim^-0.5, lse_attn.py:148)
- * bf16/fp16 q and K of one dtype with D = 128 or 64 and Hq/Hkv from 1 to 16 run on the
+ * bf16/fp16 q and K of one dtype with D = 256, 128 or 64 and Hq/Hkv from 1 to 16 run on the
  * matrix cores (groups of 3, 5-7 and 9-15 laid out as 4, 8 and 16 rows per query, the extra rows
- * padding; 512/G' queries per launch for the laid-out group G', more as several
- * launches); every other case uses float32 dot products.
+ * padding; 512/G' queries per launch for the laid-out group G', 256/G' at D = 256, more
+ * as several launches); every other case uses float32 dot products.
  */
 int actkv_action_scores(
     const void *q, int q_dtype, int64_t q_sl, int64_t q_sr, int64_t q_sn, int64_t q_sh,
@@ -299,9 +299,10 @@ size_t actkv_lrfu_workspace_size(int L, int R, int max_seq);
  *       block_table (ids outside the pool are skipped).
  * out : float32 [L, R, N, Hq, D], strides o_sl o_sr o_sn o_sh, unit last
  * lse : float32 [L, R, N, Hq], strides lse_sl lse_sr lse_sn, unit last
- * bf16/fp16 with D = 128 or 64 (any Hq/Hkv) run on the matrix cores
+ * bf16/fp16 with D = 256, 128 or 64 (any Hq/Hkv) run on the matrix cores
  * (each probability enters the P.V product as a hi and a lo term in the cache
- * dtype, P = hi + lo to about 2^-16 relative, float32 accumulation); every other
+ * dtype, P = hi + lo to about 2^-16 relative, at D = 256 in bf16 a third term,
+ * float32 accumulation); every other
  * case uses float32 dot products.  D <= 512.
  * workspace: optional, actkv_paged_attention_workspace_size(...) bytes, any
  * contents.  With it, long sequences are split into token chunks attended in
