@@ -22,7 +22,7 @@
 // span both halves of a wave, and their max is taken across the halves.  Groups of
 // 3, 5-7 and 9-15 take that kernel too, laid out as 4, 8 and 16 rows per query
 // (padding rows load no query and start at -inf).  The generic kernels cover every
-// other shape/dtype (fp32 caches or queries, head dims other than 64 and 128, groups
+// other shape/dtype (fp32 caches or queries, head dims other than 64, 128 and 256, groups
 // above 16, blocks that are not a power of two from 16 up) in float32 and follow the
 // reference fold order exactly: for each query in turn,
 // out += (p - out) / (n_seen + n + 1).  score_generic_rows_kernel (head dims that are a
@@ -38,7 +38,7 @@
 namespace actkv {
 
 // Longest token range of one MFMA workgroup (its block-table slice holds
-// MFMA_MAX_TOKENS / 16 entries, one per thread of the 512).
+// MFMA_MAX_TOKENS / 16 entries, one or two per thread).
 constexpr int MFMA_MAX_TOKENS = 8192;
 
 struct ScoreArgs {
@@ -616,19 +616,28 @@ score_kslice_kernel(ScoreArgs a, int tpw, int cpp, int pairs, int bs_shift) {
 // tile.  Per-token partial sums (one per row group and lane half) go to LDS at
 // the end of the chunk; after the next barrier the first HP x CH threads add each
 // head's in a fixed order and write the running means.
+//
+// Head dim 256 runs the same kernel with 4 waves, one per SIMD: a wave's 64 query rows are 128
+// registers there, and with the two fragment buffers they leave no room for a second wave.  A
+// launch takes 256 rows (two row groups of 64 up to 128 rows, four above), chunks of 64 tokens,
+// two in flight.  One 32k-token layer, 128 queries, 16 query heads over 8 KV heads, bf16: 57 us,
+// against 546 us on the float32 kernel this head dim took before; 48 fp16 queries over 5000 and
+// 3333 tokens 26 us against 148; scores 2.2e-7 from 64 bits, against 2.6e-7.
+constexpr int qreg_waves(int dh) { return dh == 256 ? 4 : 8; }
 template <typename T, typename V8, int G, bool CAUSAL, int RG, int NBUF, bool SWZ, int CH, int HP, int DH = 128>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(qreg_waves(DH) * 64)
+__attribute__((amdgpu_waves_per_eu(qreg_waves(DH) / 4, qreg_waves(DH) / 4)))
 score_qreg_kernel(ScoreArgs a, int tpw, int cpp, int pairs, int bs_shift) {
   // QG: queries in an aligned group of four output rows (G <= 4); with G = 8 a query's
   // heads span two such groups, one in each half of the wave, with G = 16 four (two in
   // each half)
-  constexpr int NW = 8, TG = NW / RG, KS = DH / 16, QG = G >= 4 ? 1 : 4 / G;
-  static_assert(DH == 64 || DH == 128, "head dims");
+  constexpr int NW = qreg_waves(DH), TG = NW / RG, KS = DH / 16, QG = G >= 4 ? 1 : 4 / G;
+  static_assert(DH == 64 || DH == 128 || DH == 256, "head dims");
   constexpr int PB = DH * 2;            // bytes of one head's piece of a token row
   constexpr int NC = PB / 16;           // its 16-byte columns
-  constexpr int NCS = NC == 16 ? 4 : 3;  // log2(NC)
+  constexpr int NCS = NC == 32 ? 5 : NC == 16 ? 4 : 3;  // log2(NC)
   static_assert(G == 1 || G == 2 || G == 4 || G == 8 || G == 16, "group sizes");
-  static_assert(RG == 2 || RG == 4 || RG == 8, "row groups");
+  static_assert((RG == 2 || RG == 4 || RG == 8) && RG <= NW, "row groups");
   static_assert(HP == 1 || HP == 2 || HP == 4 || HP == 8, "heads per workgroup");
   static_assert(RG % HP == 0 && (HP == 1 || SWZ), "whole row groups per head; packed heads use rows");
   static_assert(NBUF >= 2 && NBUF <= 4, "K chunk buffers");
@@ -696,8 +705,11 @@ score_qreg_kernel(ScoreArgs a, int tpw, int cpp, int pairs, int bs_shift) {
 
   // ---- set-up: every load goes out before the first wait
   const int b0 = t_begin >> bs_shift;
-  const int nbt = ((t_end - 1) >> bs_shift) - b0 + 1;  // <= 512: one entry per thread
-  const int bt_own = a.bt[(int64_t)r * a.bt_sr + b0 + min(tid, nbt - 1)];
+  const int nbt = ((t_end - 1) >> bs_shift) - b0 + 1;  // <= 512: BTN entries per thread
+  constexpr int BTN = MFMA_MAX_TOKENS / 16 / (NW * 64);
+  int bt_own[BTN];
+#pragma unroll
+  for (int i = 0; i < BTN; ++i) bt_own[i] = a.bt[(int64_t)r * a.bt_sr + b0 + min(tid + i * NW * 64, nbt - 1)];
   V8 af[2][KS];
   f32x16 seed[2];
   int lim[2][4][QG];
@@ -761,7 +773,9 @@ score_qreg_kernel(ScoreArgs a, int tpw, int cpp, int pairs, int bs_shift) {
       }
     }
   }
-  if (tid < nbt) bts[tid] = (bt_own >= 0 && bt_own < a.num_blocks) ? bt_own : -1;
+#pragma unroll
+  for (int i = 0; i < BTN; ++i)
+    if (tid + i * NW * 64 < nbt) bts[tid + i * NW * 64] = (bt_own[i] >= 0 && bt_own[i] < a.num_blocks) ? bt_own[i] : -1;
   // every set-up load has landed: the chunk loop's counts of vector memory operations
   // start from zero, and no later wait for the query tile drains the chunk loads
   __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -1100,7 +1114,7 @@ template <typename T, typename V8, int G, int DH = 128>
 static int launch_mfma(const ScoreArgs &a0, int bs_shift, hipStream_t st) {
   const int pairs = a0.L * a0.R * a0.Hkv;
   const int span = a0.max_blocks * a0.BS;
-  const int q_per_launch = 512 / G;  // both kernels take at most 512 query rows
+  const int q_per_launch = qreg_waves(DH) * 64 / G;  // query rows of a launch: 64 per wave
   const bool causal = a0.kv_len != nullptr;
   const int choice = mfma_choice();
   for (int qc0 = 0; qc0 < a0.N; qc0 += q_per_launch) {
@@ -1129,10 +1143,10 @@ static int launch_mfma(const ScoreArgs &a0, int bs_shift, hipStream_t st) {
     const int grid = ((packs + 7) / 8) * 8 * cpp;                                                  \
     if (causal)                                                                                    \
       hipLaunchKernelGGL((score_qreg_kernel<T, V8, G, true, RGV, NB, SW, CHV, HPV, DH>), dim3(grid), \
-                         dim3(512), 0, st, a, tpw, cpp, packs, bs_shift);                          \
+                         dim3(qreg_waves(DH) * 64), 0, st, a, tpw, cpp, packs, bs_shift);          \
     else                                                                                           \
       hipLaunchKernelGGL((score_qreg_kernel<T, V8, G, false, RGV, NB, SW, CHV, HPV, DH>), dim3(grid),\
-                         dim3(512), 0, st, a, tpw, cpp, packs, bs_shift);                          \
+                         dim3(qreg_waves(DH) * 64), 0, st, a, tpw, cpp, packs, bs_shift);          \
   } while (0)
       // Up to 128 rows the call streams K at the HBM rate.  Several KV heads of the same
       // tokens then share a workgroup (8 up to 64 rows, 4 up to 128): every wave keeps 64
@@ -1142,7 +1156,10 @@ static int launch_mfma(const ScoreArgs &a0, int bs_shift, hipStream_t st) {
       // rows the matrix cores bound it: fragment layout (fewer address instructions) and
       // two chunks in flight.  Set-up measured at ~5 us against ~3.7 us per 512-row chunk
       // of 128 tokens.
-      if constexpr (G >= 8) {
+      if constexpr (DH == 256) {
+        if (rows <= 128) ACTKV_QREG(2, 3, true, 64, 2.0, 1);
+        else ACTKV_QREG(4, 3, true, 64, 2.0, 1);
+      } else if constexpr (G >= 8) {
         if (rows <= 128) ACTKV_QREG(2, 3, true, 128, 1.5, 1);
         else if (rows <= 256) ACTKV_QREG(4, 3, true, 128, 1.5, 1);
         else ACTKV_QREG(8, 2, false, 128, 1.5, 1);
@@ -1284,16 +1301,18 @@ extern "C" int actkv_action_scores(
   for (int sh = 4; sh < 31; ++sh)
     if (block_size == (1 << sh)) bs_shift = sh;
   const bool mfma_ok = q_dtype == kv_dtype && (kv_dtype == ACTKV_BF16 || kv_dtype == ACTKV_F16) &&
-                       (D == 128 || D == 64) && G >= 1 && G <= 16 && scale > 0.f && vec_ok &&
+                       (D == 256 || D == 128 || D == 64) && G >= 1 && G <= 16 && scale > 0.f && vec_ok &&
                        bs_shift >= 0;
   int rc;
   if (mfma_ok) {
     if (kv_dtype == ACTKV_BF16)
-      rc = D == 64 ? launch_mfma_groups<__bf16, bf16x8, 64>(a, G, bs_shift, st)
-                   : launch_mfma_groups<__bf16, bf16x8, 128>(a, G, bs_shift, st);
+      rc = D == 64    ? launch_mfma_groups<__bf16, bf16x8, 64>(a, G, bs_shift, st)
+           : D == 128 ? launch_mfma_groups<__bf16, bf16x8, 128>(a, G, bs_shift, st)
+                      : launch_mfma_groups<__bf16, bf16x8, 256>(a, G, bs_shift, st);
     else
-      rc = D == 64 ? launch_mfma_groups<_Float16, f16x8, 64>(a, G, bs_shift, st)
-                   : launch_mfma_groups<_Float16, f16x8, 128>(a, G, bs_shift, st);
+      rc = D == 64    ? launch_mfma_groups<_Float16, f16x8, 64>(a, G, bs_shift, st)
+           : D == 128 ? launch_mfma_groups<_Float16, f16x8, 128>(a, G, bs_shift, st)
+                      : launch_mfma_groups<_Float16, f16x8, 256>(a, G, bs_shift, st);
   } else {
     switch (q_dtype) {
       case ACTKV_F32: rc = dispatch_generic_kv<float>(a, kv_dtype, st); break;
