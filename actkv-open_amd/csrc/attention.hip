@@ -247,6 +247,51 @@ __device__ __forceinline__ int dswz(int t) {
 
 typedef short dv4s __attribute__((ext_vector_type(4)));
 
+// Two floats rounded to T in one dword (one v_cvt_pk on gfx950; element-wise conversions take one
+// each), and the two values of such a dword.
+template <typename T>
+__device__ __forceinline__ uint32_t pack2(float x, float y) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef T t2 __attribute__((ext_vector_type(2)));
+  const f2 v = {x, y};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, t2));
+}
+template <typename T>
+__device__ __forceinline__ float2 unpack2(uint32_t u) {
+  if constexpr (__is_same(T, __bf16)) {
+    return make_float2(__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u));
+  } else {
+    typedef T t2 __attribute__((ext_vector_type(2)));
+    const t2 v = __builtin_bit_cast(t2, u);
+    return make_float2((float)v[0], (float)v[1]);
+  }
+}
+
+// The probabilities of a 32-token slice, p[16] per lane, as TERMS operands of the cache dtype for
+// each 16-token k step: p = term 0 + term 1 (+ term 2), each the rest rounded.
+template <typename T, typename V8, int TERMS>
+__device__ __forceinline__ void split_p(const float (&p)[16], V8 (&out)[TERMS][2]) {
+  uint32_t w[TERMS][8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    float x = p[2 * i], y = p[2 * i + 1];
+#pragma unroll
+    for (int k = 0; k < TERMS; ++k) {
+      w[k][i] = pack2<T>(x, y);
+      if (k + 1 < TERMS) {
+        const float2 r = unpack2<T>(w[k][i]);
+        x -= r.x;
+        y -= r.y;
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < TERMS; ++k)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+      out[k][b] = __builtin_bit_cast(V8, make_uint4(w[k][4 * b], w[k][4 * b + 1], w[k][4 * b + 2], w[k][4 * b + 3]));
+}
+
 template <typename T, typename V8, int DH, bool CAUSAL>
 __global__ void __launch_bounds__(DW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 attn_decode_kernel(AttnArgs a, int pairs, int bs_shift) {
@@ -377,15 +422,14 @@ attn_decode_kernel(AttnArgs a, int pairs, int bs_shift) {
     const float msafe = m_new == -INFINITY ? 0.f : m_new;
     const float alpha = __builtin_amdgcn_exp2f(m2 - msafe);
     float ps = 0.f;
-    V8 pb[2], pbl[2];  // P = hi + lo, both in the cache dtype (hi/lo split below)
+    float pe[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const float pe = __builtin_amdgcn_exp2f(fmaf(st[e], c2, -msafe));
-      ps += pe;
-      const T hi = (T)pe;
-      pb[e >> 3][e & 7] = hi;
-      pbl[e >> 3][e & 7] = (T)(pe - (float)hi);
+      pe[e] = __builtin_amdgcn_exp2f(fmaf(st[e], c2, -msafe));
+      ps += pe[e];
     }
+    V8 pt[2][2];  // P = hi + lo, both in the cache dtype
+    split_p<T, V8, 2>(pe, pt);
     {
       const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(ps), __float_as_uint(ps), false, false);
       ps = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
@@ -419,11 +463,11 @@ attn_decode_kernel(AttnArgs a, int pairs, int bs_shift) {
         const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
         const V8 va = __builtin_bit_cast(V8, make_uint4(l2.x, l2.y, h2.x, h2.y));
         if constexpr (__is_same(T, __bf16)) {
-          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pb[kb], oacc[dt], 0, 0, 0);
-          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pbl[kb], oacc[dt], 0, 0, 0);
+          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pt[0][kb], oacc[dt], 0, 0, 0);
+          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pt[1][kb], oacc[dt], 0, 0, 0);
         } else {
-          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pb[kb], oacc[dt], 0, 0, 0);
-          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pbl[kb], oacc[dt], 0, 0, 0);
+          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pt[0][kb], oacc[dt], 0, 0, 0);
+          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pt[1][kb], oacc[dt], 0, 0, 0);
         }
       }
     }
@@ -586,7 +630,8 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
   // bf16 at head dim 256: a third term gives P 24 significant bits, as many as the float32 path
   // that serves the other dtypes there (with hi + lo alone out was 1.3e-6 from 64 bits on
   // causal prefill against that path's 7.7e-7)
-  constexpr bool P3 = DH == 256 && __is_same(T, __bf16);
+  constexpr int PT = DH == 256 && __is_same(T, __bf16) ? 3 : 2;
+  static_assert(NSTG == 2, "the fragment addresses alternate between two ring slots");
   static_assert((2 * SH::IPP) % NW == 0, "whole load instructions per wave");
   __shared__ __attribute__((aligned(1024))) unsigned char ring[NSTG][SH::SBYTES];
   __shared__ int tbl[TBLW];
@@ -683,24 +728,36 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
   const uint64_t vbase = kbase + (uint64_t)a.kv_sv * sizeof(T);
   const unsigned blk_bytes = (unsigned)(((int64_t)(BS - 1) * a.kv_ss + DH) * sizeof(T));
   const unsigned ring_base = (unsigned)(uintptr_t)&ring[0][0];
+  // The stage's table entries come in one LDS read (lane i holds instruction i's; read one by one
+  // between the loads they cost an LDS round trip each), and a lane's offset is a row's part, the
+  // same for every instruction up to a scalar, plus its chunk: RPI divides the block size, so an
+  // instruction's rows are consecutive rows of one block, and dswz of row RPI tg + i is
+  // dswz(RPI tg) ^ dswz(i).
+  const int lrow = lane >> NCS;
+  const int c_lane = (lane & (NC - 1)) ^ dswz<DH>(lrow);
+  const unsigned ss_bytes = (unsigned)(a.kv_ss * (int64_t)sizeof(T));   // a block spans less than 4 GiB
+  const unsigned row_off = (unsigned)lrow * ss_bytes;
+  const uint64_t sb_bytes = (uint64_t)a.kv_sb * sizeof(T);
+  const int tg_lane = (wave * PER + min(lane, PER - 1)) % SH::IPP;
   auto issue = [&](int gi) {
+    const int phv = tbl[((c_begin + gi * ST + RPI * tg_lane) >> bs_shift) - blk0 - wbase];
+    const bool whole = gi * ST + ST <= S;                    // every token of the stage exists
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int k = wave * PER + i;
       const int plane = k / SH::IPP, tg = k % SH::IPP;
       const int t0 = gi * ST + RPI * tg;                     // chunk-relative first token
-      const int bi = ((c_begin + t0) >> bs_shift) - blk0 - wbase;
-      const int ph = __builtin_amdgcn_readfirstlane(tbl[bi]);
-      const uint64_t bb = (plane ? vbase : kbase) + (uint64_t)(ph < 0 ? 0 : ph) * (uint64_t)a.kv_sb * sizeof(T);
+      const int ph = __builtin_amdgcn_readlane(phv, i);
+      const uint64_t bb = (plane ? vbase : kbase) + (uint64_t)(ph < 0 ? 0 : ph) * sb_bytes;
       ri32x4 rs;
       rs[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)bb);
       rs[1] = __builtin_amdgcn_readfirstlane((int)((uint32_t)(bb >> 32) & 0xffffu));
       rs[2] = __builtin_amdgcn_readfirstlane(ph < 0 ? 0 : (int)blk_bytes);
       rs[3] = 0x00020000;
-      const int tl = RPI * tg + (lane >> NCS);               // token within the stage
-      const int t = gi * ST + tl;
-      const int c = (lane & (NC - 1)) ^ dswz<DH>(tl);         // global chunk landing in slot lane%NC
-      const unsigned voff = t < S ? (unsigned)((((c_begin + t) & (BS - 1)) * a.kv_ss + c * 8) * sizeof(T)) : 0xfffffff0u;
+      const unsigned s_row = (unsigned)((c_begin + t0) & (BS - 1)) * ss_bytes;
+      // the global chunk landing in slot lane % NC of the row
+      unsigned voff = row_off + s_row + (unsigned)((c_lane ^ dswz<DH>(RPI * tg)) << 4);
+      if (!whole) voff = t0 + lrow < S ? voff : 0xfffffff0u;
       const unsigned dst = ring_base + (unsigned)((gi % NSTG) * SH::SBYTES + plane * ST * PB + tg * 1024);
       buf_lds16(rs, voff, __builtin_amdgcn_readfirstlane(dst));
     }
@@ -722,15 +779,29 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
   const int jq = (lane & 15) >> 2, qq = lane & 3;
   const int dgrp = 16 * ((lane >> 4) & 1) + 4 * qq;
   struct Tiles { f32x16 s[RT]; };
-  // S^T = K . Q^T of one 32-token slice for every row tile: each K fragment read once
-  auto qk = [&](const unsigned char *kl) {
+  // LDS addresses of this lane's fragments in the stage being multiplied: one per k step (K rows)
+  // and two per output tile (V rows, tokens of j and j + 8); slices and k steps of 16 tokens are
+  // constant offsets from them (computed per slice they took 27 VALU operations each)
+  typedef const __attribute__((address_space(3))) unsigned char *lds_ptr;
+  lds_ptr ka[KS], va_lo[DT], va_hi[DT];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+    ka[ks] = (lds_ptr)&ring[0][0] + (lcol * PB + (((2 * ks + lh) ^ dswz<DH>(lcol)) << 4));
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) {
+    const int d = 32 * dt + dgrp, cc = d >> 3, half = (d >> 2) & 1;
+    const int t_lo = 4 * lh + jq, t_hi = t_lo + 8;
+    va_lo[dt] = (lds_ptr)&ring[0][0] + (ST * PB + t_lo * PB + ((cc ^ dswz<DH>(t_lo)) << 4) + half * 8);
+    va_hi[dt] = (lds_ptr)&ring[0][0] + (ST * PB + t_hi * PB + ((cc ^ dswz<DH>(t_hi)) << 4) + half * 8);
+  }
+  // S^T = K . Q^T of 32-token slice b for every row tile: each K fragment read once
+  auto qk = [&](int b) {
     Tiles st;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) st.s[rt] = f32x16{};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      const int c = 2 * ks + lh;
-      const V8 kf = *(const V8 *)(kl + lcol * PB + ((c ^ dswz<DH>(lcol)) << 4));
+      const V8 kf = *(const __attribute__((address_space(3))) V8 *)(ka[ks] + b * 32 * PB);
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
         if constexpr (__is_same(T, __bf16))
@@ -743,8 +814,8 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
   };
   // online softmax of each tile's rows over the slice, then O^T += V^T . P^T with each V^T
   // fragment read once for all tiles
-  auto softmax_pv = [&](Tiles &st, const unsigned char *vl, int t0) {
-    V8 pb[RT][2], pbl[RT][2], pbm[RT][2];  // P = hi + lo (+ a third term), in the cache dtype
+  auto softmax_pv = [&](Tiles &st, int b, int t0) {
+    V8 pt[RT][PT][2];  // P as PT terms in the cache dtype
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       f32x16 &x = st.s[rt];
@@ -766,17 +837,13 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
       const float msafe = m_new == -INFINITY ? 0.f : m_new;
       const float alpha = __builtin_amdgcn_exp2f(m2[rt] - msafe);
       float ps = 0.f;
+      float pe[16];
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const float pe = __builtin_amdgcn_exp2f(fmaf(x[e], c2, -msafe));
-        ps += pe;
-        const T hi = (T)pe;
-        pb[rt][e >> 3][e & 7] = hi;
-        const float res = pe - (float)hi;
-        const T lo = (T)res;
-        pbl[rt][e >> 3][e & 7] = lo;
-        if constexpr (P3) pbm[rt][e >> 3][e & 7] = (T)(res - (float)lo);
+        pe[e] = __builtin_amdgcn_exp2f(fmaf(x[e], c2, -msafe));
+        ps += pe[e];
       }
+      split_p<T, V8, PT>(pe, pt[rt]);
       {
         const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(ps), __float_as_uint(ps), false, false);
         ps = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
@@ -795,25 +862,20 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
     for (int kb = 0; kb < 2; ++kb) {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
-        const int d = 32 * dt + dgrp;
-        const int cc = d >> 3, half = (d >> 2) & 1;
-        const int t_lo = 16 * kb + 4 * lh + jq, t_hi = t_lo + 8;
         const dv4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (dv4s __attribute__((address_space(3))) *)(vl + t_lo * PB + ((cc ^ dswz<DH>(t_lo)) << 4) + half * 8));
+            (dv4s __attribute__((address_space(3))) *)(va_lo[dt] + (b * 32 + 16 * kb) * PB));
         const dv4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (dv4s __attribute__((address_space(3))) *)(vl + t_hi * PB + ((cc ^ dswz<DH>(t_hi)) << 4) + half * 8));
+            (dv4s __attribute__((address_space(3))) *)(va_hi[dt] + (b * 32 + 16 * kb) * PB));
         const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
         const V8 va = __builtin_bit_cast(V8, make_uint4(l2.x, l2.y, h2.x, h2.y));
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
-          if constexpr (__is_same(T, __bf16)) {
-            oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pb[rt][kb], oacc[rt][dt], 0, 0, 0);
-            oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pbl[rt][kb], oacc[rt][dt], 0, 0, 0);
-            if constexpr (P3)
-              oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pbm[rt][kb], oacc[rt][dt], 0, 0, 0);
-          } else {
-            oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pb[rt][kb], oacc[rt][dt], 0, 0, 0);
-            oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pbl[rt][kb], oacc[rt][dt], 0, 0, 0);
+#pragma unroll
+          for (int k = 0; k < PT; ++k) {
+            if constexpr (__is_same(T, __bf16))
+              oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pt[rt][k][kb], oacc[rt][dt], 0, 0, 0);
+            else
+              oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pt[rt][k][kb], oacc[rt][dt], 0, 0, 0);
           }
         }
       }
@@ -836,18 +898,22 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
       ensure_window(gi);
       issue(gi);
     }
-    const unsigned char *kl = ring[gs % NSTG];
-    const unsigned char *vl = kl + ST * PB;
     // the next slice's S^T chain is issued before this slice's softmax, so the matrix
     // core works while the VALU does the exp/max/sum
-    Tiles st_cur = qk(kl);
+    Tiles st_cur = qk(0);
 #pragma unroll
     for (int b = 0; b < ST / 32; ++b) {
       Tiles st_next;
-      if (b + 1 < ST / 32) st_next = qk(kl + (b + 1) * 32 * PB);
-      softmax_pv(st_cur, vl + b * 32 * PB, gs * ST + 32 * b);
+      if (b + 1 < ST / 32) st_next = qk(b + 1);
+      softmax_pv(st_cur, b, gs * ST + 32 * b);
       st_cur = st_next;
     }
+    // the lane's addresses move to the other ring slot
+    const int hop = gs & 1 ? -SH::SBYTES : SH::SBYTES;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) ka[ks] += hop;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) { va_lo[dt] += hop; va_hi[dt] += hop; }
   }
 
 #pragma unroll
