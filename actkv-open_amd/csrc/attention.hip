@@ -41,9 +41,9 @@
 // Head dim 256 runs the ring kernel for every row count, one wave per SIMD (a wave's O tile is 128
 // registers, its query rows 64), with P as three terms in bf16.  16 query heads over 8 KV heads
 // in bf16, against the float32 path these shapes took before: 24 causal queries over 12000 and
-// 5003 tokens, attention and scoring together, 742 -> 102 us; a decode step over 8 x 8k tokens
-// 310 -> 182 us; 700 causal queries over 3000 and 2003 tokens 2555 -> 266 us.  out is 5.5e-7 to
-// 6.9e-7 from 64 bits on them, against 7.7e-7 to 9.1e-7.
+// 5003 tokens, attention and scoring together, 742 -> 91 us; a decode step over 8 x 8k tokens
+// 318 -> 121 us; 700 causal queries over 3000 and 2003 tokens 2567 -> 224 us.  out is 5.5e-7 to
+// 6.9e-7 from 64 bits on them, against 7.7e-7 to 9.9e-7.
 //
 // Generic path (any other dtype / head_dim up to 512 / block size): float32, up to 8
 // query rows of one KV head per workgroup (a decode step's GQA group of up to 8 heads
@@ -248,7 +248,7 @@ __device__ __forceinline__ int dswz(int t) {
 typedef short dv4s __attribute__((ext_vector_type(4)));
 
 // Two floats rounded to T in one dword (one v_cvt_pk on gfx950; element-wise conversions take one
-// each), and the two values of such a dword.
+// each).
 template <typename T>
 __device__ __forceinline__ uint32_t pack2(float x, float y) {
   typedef float f2 __attribute__((ext_vector_type(2)));
@@ -256,21 +256,32 @@ __device__ __forceinline__ uint32_t pack2(float x, float y) {
   const f2 v = {x, y};
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, t2));
 }
-template <typename T>
-__device__ __forceinline__ float2 unpack2(uint32_t u) {
-  if constexpr (__is_same(T, __bf16)) {
-    return make_float2(__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u));
-  } else {
-    typedef T t2 __attribute__((ext_vector_type(2)));
-    const t2 v = __builtin_bit_cast(t2, u);
-    return make_float2((float)v[0], (float)v[1]);
-  }
+
+// x - (low half of u) and x - (high half of u), both halves of type T: one dot product each in
+// bf16 (the difference is exact where u is x rounded).  The constants (-1, 0) and (0, -1) come in
+// registers: as a literal, 0x0000bf80 is assembled to the inline constant -1.0, which the dot
+// product reads as 0xbf800000.
+struct MinusOne { uint32_t lo, hi; };
+__device__ __forceinline__ MinusOne minus_one() {
+  MinusOne m;
+  asm("s_mov_b32 %0, 0xbf80" : "=s"(m.lo));
+  asm("s_mov_b32 %0, 0xbf800000" : "=s"(m.hi));
+  return m;
+}
+__device__ __forceinline__ float minus_half(float x, uint32_t u, uint32_t m, int, __bf16) {
+  typedef __bf16 t2 __attribute__((ext_vector_type(2)));
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(t2, u), __builtin_bit_cast(t2, m), x, false);
+}
+__device__ __forceinline__ float minus_half(float x, uint32_t u, uint32_t, int half, _Float16) {
+  typedef _Float16 t2 __attribute__((ext_vector_type(2)));
+  return x - (float)__builtin_bit_cast(t2, u)[half];
 }
 
-// The probabilities of a 32-token slice, p[16] per lane, as TERMS operands of the cache dtype for
-// each 16-token k step: p = term 0 + term 1 (+ term 2), each the rest rounded.
-template <typename T, typename V8, int TERMS>
-__device__ __forceinline__ void split_p(const float (&p)[16], V8 (&out)[TERMS][2]) {
+// The probabilities of a 32-token slice, p[16] per lane, as TERMS operands of the cache dtype
+// (eight values in four registers) for each 16-token k step: p = term 0 + term 1 (+ term 2),
+// each the rest rounded.
+template <typename T, int TERMS>
+__device__ __forceinline__ void split_p(const float (&p)[16], uint4 (&out)[TERMS][2], MinusOne m1) {
   uint32_t w[TERMS][8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
@@ -279,9 +290,8 @@ __device__ __forceinline__ void split_p(const float (&p)[16], V8 (&out)[TERMS][2
     for (int k = 0; k < TERMS; ++k) {
       w[k][i] = pack2<T>(x, y);
       if (k + 1 < TERMS) {
-        const float2 r = unpack2<T>(w[k][i]);
-        x -= r.x;
-        y -= r.y;
+        x = minus_half(x, w[k][i], m1.lo, 0, T{});
+        y = minus_half(y, w[k][i], m1.hi, 1, T{});
       }
     }
   }
@@ -289,7 +299,7 @@ __device__ __forceinline__ void split_p(const float (&p)[16], V8 (&out)[TERMS][2
   for (int k = 0; k < TERMS; ++k)
 #pragma unroll
     for (int b = 0; b < 2; ++b)
-      out[k][b] = __builtin_bit_cast(V8, make_uint4(w[k][4 * b], w[k][4 * b + 1], w[k][4 * b + 2], w[k][4 * b + 3]));
+      out[k][b] = make_uint4(w[k][4 * b], w[k][4 * b + 1], w[k][4 * b + 2], w[k][4 * b + 3]);
 }
 
 template <typename T, typename V8, int DH, bool CAUSAL>
@@ -384,6 +394,7 @@ attn_decode_kernel(AttnArgs a, int pairs, int bs_shift) {
   };
 
   const float c2 = a.scale * 1.4426950408889634f;
+  const MinusOne m1 = minus_one();
   float m2 = -INFINITY, lsum = 0.f;
   f32x16 oacc[DT];
 #pragma unroll
@@ -428,8 +439,8 @@ attn_decode_kernel(AttnArgs a, int pairs, int bs_shift) {
       pe[e] = __builtin_amdgcn_exp2f(fmaf(st[e], c2, -msafe));
       ps += pe[e];
     }
-    V8 pt[2][2];  // P = hi + lo, both in the cache dtype
-    split_p<T, V8, 2>(pe, pt);
+    uint4 pt[2][2];  // P = hi + lo, both in the cache dtype
+    split_p<T, 2>(pe, pt, m1);
     {
       const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(ps), __float_as_uint(ps), false, false);
       ps = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
@@ -463,11 +474,11 @@ attn_decode_kernel(AttnArgs a, int pairs, int bs_shift) {
         const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
         const V8 va = __builtin_bit_cast(V8, make_uint4(l2.x, l2.y, h2.x, h2.y));
         if constexpr (__is_same(T, __bf16)) {
-          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pt[0][kb], oacc[dt], 0, 0, 0);
-          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pt[1][kb], oacc[dt], 0, 0, 0);
+          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(V8, pt[0][kb]), oacc[dt], 0, 0, 0);
+          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, __builtin_bit_cast(V8, pt[1][kb]), oacc[dt], 0, 0, 0);
         } else {
-          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pt[0][kb], oacc[dt], 0, 0, 0);
-          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pt[1][kb], oacc[dt], 0, 0, 0);
+          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, __builtin_bit_cast(V8, pt[0][kb]), oacc[dt], 0, 0, 0);
+          oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, __builtin_bit_cast(V8, pt[1][kb]), oacc[dt], 0, 0, 0);
         }
       }
     }
@@ -605,24 +616,62 @@ __device__ __forceinline__ void wait_stages(int rem) {
 
 typedef int ri32x4 __attribute__((ext_vector_type(4)));
 
-// 16 bytes from buffer `rsrc` at byte offset voff into LDS at lds_base + 16 * lane.
-// Inline assembly: the compiler's wait counting would otherwise drain every load in
-// flight before each LDS read of the ring; the kernel counts them itself.  M0 carries
-// the LDS base and is restored.
-__device__ __forceinline__ void buf_lds16(ri32x4 rsrc, unsigned voff, unsigned lds_base) {
+// N loads of 16 bytes per lane from buffer `rsrc`, at byte offsets voff[i], into LDS at
+// lds_base + 1024 i + 16 * lane.  Inline assembly: the compiler's wait counting would otherwise
+// drain every load in flight before each LDS read of the ring; the kernel counts them itself.
+// M0 carries the LDS base and is restored.
+template <int N>
+__device__ __forceinline__ void buf_lds16(ri32x4 rsrc, const unsigned *voff, unsigned lds_base) {
+  static_assert(N % 2 == 0, "pairs of loads");
   unsigned saved;
-  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n\ts_mov_b32 m0, %0"
-               : "=&s"(saved)
-               : "v"(voff), "s"(rsrc), "s"(lds_base)
-               : "memory");
+  if constexpr (N == 2) {
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\tbuffer_load_dwordx4 %1, %3, 0 offen lds\n\t"
+                 "s_add_u32 m0, m0, 0x400\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved)
+                 : "v"(voff[0]), "v"(voff[1]), "s"(rsrc), "s"(lds_base)
+                 : "memory", "scc");
+  } else if constexpr (N == 4) {
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %6\n\tbuffer_load_dwordx4 %1, %5, 0 offen lds\n\t"
+                 "s_add_u32 m0, m0, 0x400\n\tbuffer_load_dwordx4 %2, %5, 0 offen lds\n\t"
+                 "s_add_u32 m0, m0, 0x400\n\tbuffer_load_dwordx4 %3, %5, 0 offen lds\n\t"
+                 "s_add_u32 m0, m0, 0x400\n\tbuffer_load_dwordx4 %4, %5, 0 offen lds\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved)
+                 : "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(rsrc), "s"(lds_base)
+                 : "memory", "scc");
+  } else {
+    buf_lds16<4>(rsrc, voff, lds_base);
+    buf_lds16<N - 4>(rsrc, voff + 4, lds_base + 4096);
+  }
 }
 
-template <typename T, typename V8, int DH, int NW, int RT, bool CAUSAL>
+// Issue order of a slice: MF matrix products and RD LDS reads among its VALU work (about 130
+// operations).
+template <int MF, int RD>
+__device__ __forceinline__ void slice_schedule() {
+    constexpr int PRE = RD < 4 ? RD : 4, VPM = MF >= 128 ? 1 : 128 / MF;
+  __builtin_amdgcn_sched_group_barrier(0x100, PRE, 0);     // DS read
+#pragma unroll
+  for (int i = 0; i < MF; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     // MFMA
+    if (i < RD - PRE) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x002, VPM, 0);   // VALU
+  }
+}
+
+// A row's probabilities are 2^(s - m2).  With P as three terms (24 bits) the reference m2 follows
+// the running max only when the max of some row of the tile is more than REF_SLACK ahead, and then
+// all of the tile's sums and O are rescaled: p stays below 2^8, with the same relative precision.
+// With two terms m2 is the running max itself: its token then has p = 1, which two terms hold
+// exactly, and where attention is peaked that token dominates (bf16 causal prefill 1.5e-6 from 64
+// bits, 2.4e-6 with the slack).
+constexpr float REF_SLACK = 8.0f;
+
+template <typename T, typename V8, int DH, int NW, bool CAUSAL>
 __global__ void __launch_bounds__(NW * 64)
-__attribute__((amdgpu_waves_per_eu(RT >= 2 || DH == 256 ? 1 : (NW >= 4 ? 2 : 1), RT >= 2 || DH == 256 ? 1 : 2)))
+__attribute__((amdgpu_waves_per_eu(DH == 256 ? 1 : (NW >= 4 ? 2 : 1), DH == 256 ? 1 : 2)))
 attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
   const int G = a.G;   // query heads per KV head: rows (n, g) of a tile are independent
-  using SH = RingShape<NW * RT, DH>;
+  using SH = RingShape<NW, DH>;
   using RS = RowShape<DH>;
   constexpr int PB = RS::PB, NC = RS::NC, NCS = RS::NCS, RPI = RS::RPI, KS = RS::KS, DT = RS::DT;
   constexpr int ST = SH::ST, NSTG = SH::NSTG, TBLW = SH::TBLW;
@@ -648,7 +697,7 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
   const int r = (p / a.Hkv) % a.R;
   const int l = p / (a.Hkv * a.R);
   const int nq = attn_nq(a, r);
-  if (grp * NW * RT * 32 >= nq * G) return;
+  if (grp * NW * 32 >= nq * G) return;
   const int S_all = attn_seq_len(a, r);
   if (a.nchunk > 1 && chunk * a.tpc >= S_all) return;
   const int c_begin = min(chunk * a.tpc, S_all);
@@ -658,21 +707,13 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int lcol = lane & 31, lh = lane >> 5;
-  // the wave's RT row tiles: rows ((grp * NW + wave) * RT + rt) * 32 + lcol
-  int row[RT], n[RT], g[RT], lim_m[RT];
-  bool valid[RT];
-  int my_lim = 0;
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    row[rt] = ((grp * NW + wave) * RT + rt) * 32 + lcol;
-    n[rt] = row[rt] / G;
-    g[rt] = row[rt] % G;
-    valid[rt] = n[rt] < nq;
-    const int lim = valid[rt] ? min(max(attn_lim(a, r, n[rt], S_all) - c_begin, 0), S) : 0;
-    // the masking limit: padding rows (never written) see everything, so they never force it
-    lim_m[rt] = valid[rt] ? lim : 0x7fffffff;
-    my_lim = max(my_lim, lim);
-  }
+  const int row = (grp * NW + wave) * 32 + lcol;
+  const int n = row / G, g = row % G;
+  const bool valid = n < nq;
+  const bool active = (grp * NW + wave) * 32 < nq * G;   // a wave of padding rows only loads
+  const int my_lim = valid ? min(max(attn_lim(a, r, n, S_all) - c_begin, 0), S) : 0;
+  // the masking limit: padding rows (never written) see everything, so they never force it
+  const int lim_m = valid ? my_lim : 0x7fffffff;
   int s_end = S;
   if constexpr (CAUSAL) {
     if (tid == 0) wg_lim = 0;
@@ -683,25 +724,22 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
   }
   const int nst = (s_end + ST - 1) / ST;
 
-  V8 qf[RT][KS];
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
+  V8 qf[KS];
+  {
     const T *qp = (const T *)a.q + (int64_t)l * a.q_sl + (int64_t)r * a.q_sr +
-                  (int64_t)(valid[rt] ? n[rt] : 0) * a.q_sn + (int64_t)(h * G + g[rt]) * a.q_sh + lh * 8;
+                  (int64_t)(valid ? n : 0) * a.q_sn + (int64_t)(h * G + g) * a.q_sh + lh * 8;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[rt][ks] = *(const V8 *)(qp + ks * 16);
-    if (!valid[rt]) {
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *(const V8 *)(qp + ks * 16);
+    if (!valid) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) qf[rt][ks] = V8{};
+      for (int ks = 0; ks < KS; ++ks) qf[ks] = V8{};
     }
   }
   // the query loads complete here, before the first ring load: otherwise the compiler's
   // wait for them lands inside the loop, where the hardware counter also holds the
   // ring's loads and the wait would drain them every stage
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(qf[rt][ks]));
+  for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(qf[ks]));
 
   // ---- block table window: logical blocks [blk0 + wbase, blk0 + wbase + TBLW)
   const int blk0 = c_begin >> bs_shift;
@@ -723,62 +761,66 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
     }
   };
 
-  // ---- stage loads: instruction k of a stage: plane k / IPP, tokens RPI(k % IPP) .. +RPI-1
+  // ---- stage loads: instruction k of a stage: plane k / IPP, tokens RPI(k % IPP) .. +RPI-1.
+  // The V instructions of 16 consecutive tokens lie in one block (blocks hold at least 16 tokens,
+  // stages start at a multiple of 32): they share a buffer resource that starts at the group's
+  // first row, their offsets are the same for every group, and a stage's table entries come in
+  // one LDS read (lane j holds the wave's group j).  A resource per instruction took 110 scalar
+  // and 64 vector operations a stage; this takes 45 and 5.
+  constexpr int V = 16 / RPI, GPW = PER / V, GPP = SH::IPP / V;
+  static_assert(PER % V == 0 && SH::IPP % V == 0, "whole 16-token groups per wave and plane");
   const uint64_t kbase = (uint64_t)(uintptr_t)((const T *)a.kv + (int64_t)l * a.kv_sl + (int64_t)h * a.kv_sh);
   const uint64_t vbase = kbase + (uint64_t)a.kv_sv * sizeof(T);
-  const unsigned blk_bytes = (unsigned)(((int64_t)(BS - 1) * a.kv_ss + DH) * sizeof(T));
   const unsigned ring_base = (unsigned)(uintptr_t)&ring[0][0];
-  // The stage's table entries come in one LDS read (lane i holds instruction i's; read one by one
-  // between the loads they cost an LDS round trip each), and a lane's offset is a row's part, the
-  // same for every instruction up to a scalar, plus its chunk: RPI divides the block size, so an
-  // instruction's rows are consecutive rows of one block, and dswz of row RPI tg + i is
-  // dswz(RPI tg) ^ dswz(i).
   const int lrow = lane >> NCS;
-  const int c_lane = (lane & (NC - 1)) ^ dswz<DH>(lrow);
   const unsigned ss_bytes = (unsigned)(a.kv_ss * (int64_t)sizeof(T));   // a block spans less than 4 GiB
-  const unsigned row_off = (unsigned)lrow * ss_bytes;
+  const unsigned grp_bytes = 15 * ss_bytes + PB;
   const uint64_t sb_bytes = (uint64_t)a.kv_sb * sizeof(T);
-  const int tg_lane = (wave * PER + min(lane, PER - 1)) % SH::IPP;
-  auto issue = [&](int gi) {
-    const int phv = tbl[((c_begin + gi * ST + RPI * tg_lane) >> bs_shift) - blk0 - wbase];
-    const bool whole = gi * ST + ST <= S;                    // every token of the stage exists
+  unsigned vo[V];   // the global chunk landing in slot lane % NC of row RPI v + lrow
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int k = wave * PER + i;
-      const int plane = k / SH::IPP, tg = k % SH::IPP;
-      const int t0 = gi * ST + RPI * tg;                     // chunk-relative first token
-      const int ph = __builtin_amdgcn_readlane(phv, i);
-      const uint64_t bb = (plane ? vbase : kbase) + (uint64_t)(ph < 0 ? 0 : ph) * sb_bytes;
+  for (int v = 0; v < V; ++v)
+    vo[v] = (unsigned)(RPI * v + lrow) * ss_bytes + (unsigned)(((lane & (NC - 1)) ^ dswz<DH>(RPI * v + lrow)) << 4);
+  const int g_lane = (wave * GPW + min(lane, GPW - 1)) % GPP;
+  auto issue = [&](int gi) {
+    const int phv = tbl[((c_begin + gi * ST + 16 * g_lane) >> bs_shift) - blk0 - wbase];
+    const bool whole = gi * ST + ST <= S;                    // every token of the stage exists
+    const unsigned slot = ring_base + (unsigned)((gi % NSTG) * SH::SBYTES);
+#pragma unroll
+    for (int j = 0; j < GPW; ++j) {
+      const int k = wave * GPW + j;
+      const int plane = k / GPP, tg = k % GPP;
+      const int t0 = gi * ST + 16 * tg;                      // chunk-relative first token
+      const int ph = __builtin_amdgcn_readlane(phv, j);
+      const unsigned s_row = (unsigned)((c_begin + t0) & (BS - 1)) * ss_bytes;
+      const uint64_t bb = (plane ? vbase : kbase) + (uint64_t)(ph < 0 ? 0 : ph) * sb_bytes + s_row;
       ri32x4 rs;
       rs[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)bb);
       rs[1] = __builtin_amdgcn_readfirstlane((int)((uint32_t)(bb >> 32) & 0xffffu));
-      rs[2] = __builtin_amdgcn_readfirstlane(ph < 0 ? 0 : (int)blk_bytes);
+      rs[2] = __builtin_amdgcn_readfirstlane(ph < 0 ? 0 : (int)grp_bytes);
       rs[3] = 0x00020000;
-      const unsigned s_row = (unsigned)((c_begin + t0) & (BS - 1)) * ss_bytes;
-      // the global chunk landing in slot lane % NC of the row
-      unsigned voff = row_off + s_row + (unsigned)((c_lane ^ dswz<DH>(RPI * tg)) << 4);
-      if (!whole) voff = t0 + lrow < S ? voff : 0xfffffff0u;
-      const unsigned dst = ring_base + (unsigned)((gi % NSTG) * SH::SBYTES + plane * ST * PB + tg * 1024);
-      buf_lds16(rs, voff, __builtin_amdgcn_readfirstlane(dst));
+      const unsigned dst = __builtin_amdgcn_readfirstlane(slot + (unsigned)(plane * ST * PB + tg * V * 1024));
+      if (whole) {
+        buf_lds16<V>(rs, vo, dst);
+      } else {
+        unsigned vt[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) vt[v] = t0 + RPI * v + lrow < S ? vo[v] : 0xfffffff0u;
+        buf_lds16<V>(rs, vt, dst);
+      }
     }
   };
 
   const float c2 = a.scale * 1.4426950408889634f;
-  float m2[RT], lsum[RT];
-  f32x16 oacc[RT][DT];
+  const MinusOne m1 = minus_one();
+  float m2 = -INFINITY, lsum = 0.f;
+  f32x16 oacc[DT];
 #pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    m2[rt] = -INFINITY;
-    lsum[rt] = 0.f;
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) oacc[rt][dt][e] = 0.f;
-  }
+    for (int e = 0; e < 16; ++e) oacc[dt][e] = 0.f;
 
   const int jq = (lane & 15) >> 2, qq = lane & 3;
   const int dgrp = 16 * ((lane >> 4) & 1) + 4 * qq;
-  struct Tiles { f32x16 s[RT]; };
   // LDS addresses of this lane's fragments in the stage being multiplied: one per k step (K rows)
   // and two per output tile (V rows, tokens of j and j + 8); slices and k steps of 16 tokens are
   // constant offsets from them (computed per slice they took 27 VALU operations each)
@@ -794,72 +836,67 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
     va_lo[dt] = (lds_ptr)&ring[0][0] + (ST * PB + t_lo * PB + ((cc ^ dswz<DH>(t_lo)) << 4) + half * 8);
     va_hi[dt] = (lds_ptr)&ring[0][0] + (ST * PB + t_hi * PB + ((cc ^ dswz<DH>(t_hi)) << 4) + half * 8);
   }
-  // S^T = K . Q^T of 32-token slice b for every row tile: each K fragment read once
+  // S^T = K . Q^T of the stage's 32-token slice b
   auto qk = [&](int b) {
-    Tiles st;
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) st.s[rt] = f32x16{};
+    f32x16 st = {};
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const V8 kf = *(const __attribute__((address_space(3))) V8 *)(ka[ks] + b * 32 * PB);
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt) {
-        if constexpr (__is_same(T, __bf16))
-          st.s[rt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[rt][ks], st.s[rt], 0, 0, 0);
-        else
-          st.s[rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[rt][ks], st.s[rt], 0, 0, 0);
-      }
+      if constexpr (__is_same(T, __bf16))
+        st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], st, 0, 0, 0);
+      else
+        st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[ks], st, 0, 0, 0);
     }
     return st;
   };
-  // online softmax of each tile's rows over the slice, then O^T += V^T . P^T with each V^T
-  // fragment read once for all tiles
-  auto softmax_pv = [&](Tiles &st, int b, int t0) {
-    V8 pt[RT][PT][2];  // P as PT terms in the cache dtype
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      f32x16 &x = st.s[rt];
-      if (__builtin_amdgcn_ballot_w64(lim_m[rt] < t0 + 32) != 0ull) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int t = t0 + 8 * (e >> 2) + 4 * lh + (e & 3);
-          x[e] = t < lim_m[rt] ? x[e] : -INFINITY;
-        }
-      }
-      float mx = x[0];
-#pragma unroll
-      for (int e = 1; e < 16; ++e) mx = fmaxf(mx, x[e]);
-      {
-        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-        mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-      }
-      const float m_new = fmaxf(m2[rt], mx * c2);
-      const float msafe = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = __builtin_amdgcn_exp2f(m2[rt] - msafe);
-      float ps = 0.f;
-      float pe[16];
+  // tokens past a row's limit (slice at token t0): their logits become -inf
+  auto mask = [&](f32x16 &x, int t0) {
+    if (__builtin_amdgcn_ballot_w64(lim_m < t0 + 32) != 0ull) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        pe[e] = __builtin_amdgcn_exp2f(fmaf(x[e], c2, -msafe));
-        ps += pe[e];
-      }
-      split_p<T, V8, PT>(pe, pt[rt]);
-      {
-        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(ps), __float_as_uint(ps), false, false);
-        ps = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-      }
-      lsum[rt] = lsum[rt] * alpha + ps;
-      m2[rt] = m_new;
-      // O is rescaled only when some row of the tile raised its max
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0ull) {
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) oacc[rt][dt][e] *= alpha;
+        const int t = t0 + 8 * (e >> 2) + 4 * lh + (e & 3);
+        x[e] = t < lim_m ? x[e] : -INFINITY;
       }
     }
+  };
+  // The probabilities of a slice against the rows' reference m2, as PT terms, and their sum ps.
+  // Returns whether the reference moved (for the whole wave; m_old then holds the one before).
+  auto softmax = [&](const f32x16 &x, uint4 (&pt)[PT][2], float &ps, float &m_old) {
+    float mx = x[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) mx = fmaxf(mx, x[e]);
+    {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    }
+    const float m_new = fmaxf(m2, mx * c2);
+    const bool grow = __builtin_amdgcn_ballot_w64(m_new > m2 + (PT == 3 ? REF_SLACK : 0.f)) != 0ull;
+    m_old = m2;
+    m2 = grow ? m_new : m2;
+    const float msafe = m2 == -INFINITY ? 0.f : m2;
+    float pe[16];
+    ps = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      pe[e] = __builtin_amdgcn_exp2f(fmaf(x[e], c2, -msafe));
+      ps += pe[e];
+    }
+    split_p<T, PT>(pe, pt, m1);
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(ps), __float_as_uint(ps), false, false);
+    ps = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+    // the terms are formed here, beside this slice's products, and not sunk to their use
+#pragma unroll
+    for (int k = 0; k < PT; ++k)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+        asm volatile("" : "+v"(pt[k][kb].x), "+v"(pt[k][kb].y), "+v"(pt[k][kb].z), "+v"(pt[k][kb].w));
+    return grow;
+  };
+  // O^T += V^T . P^T of slice b
+  auto pv = [&](const uint4 (&pt)[PT][2], int b) {
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
+      V8 va[DT];
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const dv4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
@@ -867,16 +904,18 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
         const dv4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
             (dv4s __attribute__((address_space(3))) *)(va_hi[dt] + (b * 32 + 16 * kb) * PB));
         const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
-        const V8 va = __builtin_bit_cast(V8, make_uint4(l2.x, l2.y, h2.x, h2.y));
+        va[dt] = __builtin_bit_cast(V8, make_uint4(l2.x, l2.y, h2.x, h2.y));
+      }
+      // one term over all output tiles before the next: consecutive products go to
+      // different accumulators
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
+      for (int k = 0; k < PT; ++k) {
 #pragma unroll
-          for (int k = 0; k < PT; ++k) {
-            if constexpr (__is_same(T, __bf16))
-              oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va, pt[rt][k][kb], oacc[rt][dt], 0, 0, 0);
-            else
-              oacc[rt][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va, pt[rt][k][kb], oacc[rt][dt], 0, 0, 0);
-          }
+        for (int dt = 0; dt < DT; ++dt) {
+          if constexpr (__is_same(T, __bf16))
+            oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[dt], __builtin_bit_cast(V8, pt[k][kb]), oacc[dt], 0, 0, 0);
+          else
+            oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[dt], __builtin_bit_cast(V8, pt[k][kb]), oacc[dt], 0, 0, 0);
         }
       }
     }
@@ -898,15 +937,45 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
       ensure_window(gi);
       issue(gi);
     }
-    // the next slice's S^T chain is issued before this slice's softmax, so the matrix
-    // core works while the VALU does the exp/max/sum
-    Tiles st_cur = qk(0);
+    // Slice b's softmax runs beside the products that do not need it: S^T of slice b + 1 and
+    // P . V of slice b - 1 (one MFMA, its LDS reads and its share of the VALU work at a time:
+    // left to the compiler, the exponentials had no MFMA beside them).  One wave can issue a VALU
+    // operation every 5 cycles and an MFMA of this shape every 32, both at once; two waves share
+    // a SIMD, oldest first, so a wave's own order decides how much of that is reached.  With
+    // padding-only waves idle, the products of one term over all output tiles in a row, the lo
+    // terms by dot products and one buffer resource per 16 tokens: 48 causal queries over 4 x 8k
+    // tokens, 36 layers, 2022 -> 1873 us; 700 over 3000 and 2003 at head dim 256 259 -> 224;
+    // decode at head dim 256 over 8 x 8k 151 -> 121.
+    constexpr int NS = ST / 32;
+    if (active) {
+      f32x16 st_cur = qk(0);
+      uint4 pt[PT][2];
 #pragma unroll
-    for (int b = 0; b < ST / 32; ++b) {
-      Tiles st_next;
-      if (b + 1 < ST / 32) st_next = qk(b + 1);
-      softmax_pv(st_cur, b, gs * ST + 32 * b);
-      st_cur = st_next;
+      for (int b = 0; b < NS; ++b) {
+        mask(st_cur, gs * ST + 32 * b);
+        f32x16 st_next;
+        uint4 pt_next[PT][2];
+        float ps, m_old;
+        if (b + 1 < NS) st_next = qk(b + 1);
+        if (b > 0) pv(pt, b - 1);
+        const bool grow = softmax(st_cur, pt_next, ps, m_old);
+        if (b == 0 && NS > 1) slice_schedule<KS, KS>();
+        else if (b + 1 < NS) slice_schedule<KS + 2 * DT * PT, KS + 4 * DT>();
+        else if (NS > 1) slice_schedule<2 * DT * PT, 4 * DT>();
+        if (grow) {
+          const float alpha = __builtin_amdgcn_exp2f(m_old - (m2 == -INFINITY ? 0.f : m2));
+          lsum *= alpha;
+#pragma unroll
+          for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) oacc[dt][e] *= alpha;
+        }
+        lsum += ps;
+        st_cur = st_next;
+#pragma unroll
+        for (int k = 0; k < PT; ++k) { pt[k][0] = pt_next[k][0]; pt[k][1] = pt_next[k][1]; }
+      }
+      pv(pt, NS - 1);
     }
     // the lane's addresses move to the other ring slot
     const int hop = gs & 1 ? -SH::SBYTES : SH::SBYTES;
@@ -916,42 +985,37 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
     for (int dt = 0; dt < DT; ++dt) { va_lo[dt] += hop; va_hi[dt] += hop; }
   }
 
-#pragma unroll
-  for (int rt = 0; rt < RT; ++rt) {
-    if (!valid[rt]) continue;
-    // ---- split: the chunk's partial (unnormalised O, max, sum) for the combine kernel
-    if (a.nchunk > 1) {
-      const int64_t pr = ((int64_t)p * a.rows_pad + row[rt]) * a.nchunk + chunk;
-      float *wo = a.ws_o + pr * DH;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          f32x4 v;
-          v[0] = oacc[rt][dt][4 * i]; v[1] = oacc[rt][dt][4 * i + 1];
-          v[2] = oacc[rt][dt][4 * i + 2]; v[3] = oacc[rt][dt][4 * i + 3];
-          *(f32x4 *)(wo + 32 * dt + 8 * i + 4 * lh) = v;
-        }
-      if (lh == 0) { a.ws_ml[pr * 2] = m2[rt]; a.ws_ml[pr * 2 + 1] = lsum[rt]; }
-      continue;
-    }
-    const float inv = lsum[rt] > 0.f ? 1.0f / lsum[rt] : 0.f;
-    float *op = a.out + (int64_t)l * a.o_sl + (int64_t)r * a.o_sr + (int64_t)n[rt] * a.o_sn +
-                (int64_t)(h * G + g[rt]) * a.o_sh;
+  if (!valid) return;
+  // ---- split: the chunk's partial (unnormalised O, reference, sum) for the combine kernel
+  if (a.nchunk > 1) {
+    const int64_t pr = ((int64_t)p * a.rows_pad + row) * a.nchunk + chunk;
+    float *wo = a.ws_o + pr * DH;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int d0 = 32 * dt + 8 * i + 4 * lh;
         f32x4 v;
-        v[0] = oacc[rt][dt][4 * i] * inv; v[1] = oacc[rt][dt][4 * i + 1] * inv;
-        v[2] = oacc[rt][dt][4 * i + 2] * inv; v[3] = oacc[rt][dt][4 * i + 3] * inv;
-        *(f32x4 *)(op + d0) = v;
+        v[0] = oacc[dt][4 * i]; v[1] = oacc[dt][4 * i + 1]; v[2] = oacc[dt][4 * i + 2]; v[3] = oacc[dt][4 * i + 3];
+        *(f32x4 *)(wo + 32 * dt + 8 * i + 4 * lh) = v;
       }
-    if (lh == 0)
-      a.lse[(int64_t)l * a.lse_sl + (int64_t)r * a.lse_sr + (int64_t)n[rt] * a.lse_sn + h * G + g[rt]] =
-          lsum[rt] > 0.f ? (m2[rt] + __log2f(lsum[rt])) * 0.6931471805599453f : -INFINITY;
+    if (lh == 0) { a.ws_ml[pr * 2] = m2; a.ws_ml[pr * 2 + 1] = lsum; }
+    return;
   }
+  const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
+  float *op = a.out + (int64_t)l * a.o_sl + (int64_t)r * a.o_sr + (int64_t)n * a.o_sn + (int64_t)(h * G + g) * a.o_sh;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int d0 = 32 * dt + 8 * i + 4 * lh;
+      f32x4 v;
+      v[0] = oacc[dt][4 * i] * inv; v[1] = oacc[dt][4 * i + 1] * inv;
+      v[2] = oacc[dt][4 * i + 2] * inv; v[3] = oacc[dt][4 * i + 3] * inv;
+      *(f32x4 *)(op + d0) = v;
+    }
+  if (lh == 0)
+    a.lse[(int64_t)l * a.lse_sl + (int64_t)r * a.lse_sr + (int64_t)n * a.lse_sn + h * G + g] =
+        lsum > 0.f ? (m2 + __log2f(lsum)) * 0.6931471805599453f : -INFINITY;
 }
 
 // ------------------------------------------------------------------ split combine
@@ -1184,17 +1248,14 @@ __global__ void __launch_bounds__(256) attn_generic_kernel(AttnArgs a, int pairs
   }
 }
 
-// Ring workgroup shape for a pair with rtiles 32-row tiles of query rows: waves and row
-// tiles per wave.  Two tiles per wave (each K and V^T fragment read once for 64 rows)
-// needs about 500 registers, one wave per SIMD, and measured 4.86 ms against 3.40 ms for
-// one tile per wave at two waves per SIMD (36 layers x 32k x 128 queries): the second
-// wave hides more than the halved LDS reads save.
-struct RingCfg { int nw, rt; };
-static RingCfg ring_cfg(int rtiles, int D) {
-  if (rtiles == 1) return {1, 1};   // head dim 256 only
-  if (rtiles <= 2) return {2, 1};
-  if (rtiles <= 4 || D == 256) return {4, 1};
-  return {8, 1};
+// Waves of a ring workgroup for a pair with rtiles 32-row tiles of query rows.  (Two tiles per
+// wave, each K and V^T fragment read once for 64 rows, need about 500 registers, one wave per
+// SIMD, and measured 4.86 ms against 3.40 ms on 36 layers x 32k x 128 queries.)
+static int ring_waves(int rtiles, int D) {
+  if (rtiles == 1) return 1;   // head dim 256 only
+  if (rtiles <= 2) return 2;
+  if (rtiles <= 4 || D == 256) return 4;
+  return 8;
 }
 
 // Token-range split: enough (pair, row group, chunk) work items for about four rounds of
@@ -1235,8 +1296,7 @@ static AttnSplit attn_split(int pairs, int N, int G, int D, int span, int cus) {
     sp.tpc = sp.nchunk > 1 ? 0 : std::max(span, 1);
     return sp;
   }
-  const RingCfg cfg = ring_cfg(rtiles, D);
-  const int tiles = cfg.nw * cfg.rt;
+  const int tiles = ring_waves(rtiles, D);
   const int st = ring_stage(tiles, D);
   sp.ngroups = (rtiles + tiles - 1) / tiles;
   sp.rows_pad = N * G;   // only rows that exist are written and merged
@@ -1282,25 +1342,25 @@ static int launch_attn_mfma(AttnArgs a, int bs_shift, void *ws, size_t ws_bytes,
         hipLaunchKernelGGL((attn_decode_kernel<T, V8, DH, false>), dim3(grid), dim3(DW * 64), 0, st, a, pairs, bs_shift);
     }
   } else {
-#define ACTKV_ATTN(NWV, RTV)                                                                       \
+#define ACTKV_ATTN(NWV)                                                                            \
   do {                                                                                             \
     const int grid = ((pairs + 7) / 8) * 8 * sp.ngroups * sp.nchunk;                               \
     if (causal)                                                                                    \
-      hipLaunchKernelGGL((attn_ring_kernel<T, V8, DH, NWV, RTV, true>), dim3(grid), dim3(NWV * 64), \
+      hipLaunchKernelGGL((attn_ring_kernel<T, V8, DH, NWV, true>), dim3(grid), dim3(NWV * 64), \
                          0, st, a, pairs, sp.ngroups, bs_shift);                                   \
     else                                                                                           \
-      hipLaunchKernelGGL((attn_ring_kernel<T, V8, DH, NWV, RTV, false>), dim3(grid), dim3(NWV * 64),\
+      hipLaunchKernelGGL((attn_ring_kernel<T, V8, DH, NWV, false>), dim3(grid), dim3(NWV * 64),\
                          0, st, a, pairs, sp.ngroups, bs_shift);                                   \
   } while (0)
-  const RingCfg cfg = ring_cfg(rtiles, DH);
-  if (cfg.nw == 2) {
-    ACTKV_ATTN(2, 1);
+  const int nw = ring_waves(rtiles, DH);
+  if (nw == 2) {
+    ACTKV_ATTN(2);
   } else if constexpr (DH == 256) {
-    if (cfg.nw == 1) ACTKV_ATTN(1, 1);
-    else ACTKV_ATTN(4, 1);
+    if (nw == 1) ACTKV_ATTN(1);
+    else ACTKV_ATTN(4);
   } else {
-    if (cfg.nw == 4) ACTKV_ATTN(4, 1);
-    else ACTKV_ATTN(8, 1);
+    if (nw == 4) ACTKV_ATTN(4);
+    else ACTKV_ATTN(8);
   }
 #undef ACTKV_ATTN
   }
