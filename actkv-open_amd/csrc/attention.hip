@@ -42,7 +42,7 @@
 // registers, its query rows 64), with P as three terms in bf16.  16 query heads over 8 KV heads
 // in bf16, against the float32 path these shapes took before: 24 causal queries over 12000 and
 // 5003 tokens, attention and scoring together, 742 -> 91 us; a decode step over 8 x 8k tokens
-// 318 -> 121 us; 700 causal queries over 3000 and 2003 tokens 2567 -> 224 us.  out is 5.5e-7 to
+// 318 -> 115 us; 700 causal queries over 3000 and 2003 tokens 2567 -> 225 us.  out is 5.5e-7 to
 // 6.9e-7 from 64 bits on them, against 7.7e-7 to 9.9e-7.
 //
 // Generic path (any other dtype / head_dim up to 512 / block size): float32, up to 8
@@ -52,6 +52,7 @@
 #include "common.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace actkv {
 
@@ -147,11 +148,21 @@ __device__ __forceinline__ void attn_merge_row(const AttnArgs &a, int64_t id, in
         for (int k = 0; k < DL; ++k) ov[k] += j < nc ? wj * pre[k][j] : 0.f;
       }
     }
-    const float *wc = wo + (int64_t)c0 * DH;
-    for (int j = c0 == 0 ? PRE : 0; j < min(64, nc - c0); ++j) {
-      const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j));
+    // the next chunks' rows, PRE at a time and all in flight together (one by one, 64 chunks of a
+    // head-dim-256 row cost 48 round trips)
+    for (int j0 = c0 == 0 ? PRE : 0; j0 < min(64, nc - c0); j0 += PRE) {
 #pragma unroll
-      for (int k = 0; k < DL; ++k) ov[k] += wj * wc[j * DH + 64 * k + lane];
+      for (int j = 0; j < PRE; ++j) {
+        const int jc = min(c0 + j0 + j, nc - 1);
+#pragma unroll
+        for (int k = 0; k < DL; ++k) pre[k][j] = wo[(int64_t)jc * DH + 64 * k + lane];
+      }
+#pragma unroll
+      for (int j = 0; j < PRE; ++j) {
+        const float wj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), j0 + j));   // 0 past nc
+#pragma unroll
+        for (int k = 0; k < DL; ++k) ov[k] += c0 + j0 + j < nc ? wj * pre[k][j] : 0.f;
+      }
     }
   }
   const float inv = Lsum > 0.f ? 1.0f / Lsum : 0.f;
@@ -691,7 +702,9 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
   const int xcd = bid & 7, jj = bid >> 3;
   const int per_pair = ngroups * a.nchunk;
   const int p = (jj / per_pair) * 8 + xcd;
-  const int grp = (jj % per_pair) / a.nchunk, chunk = jj % a.nchunk;
+  // causal: the last groups see the most tokens and go first, so that the launch ends on short ones
+  const int gpos = (jj % per_pair) / a.nchunk, chunk = jj % a.nchunk;
+  const int grp = CAUSAL ? ngroups - 1 - gpos : gpos;
   if (p >= pairs) return;
   const int h = p % a.Hkv;
   const int r = (p / a.Hkv) % a.R;
@@ -1258,9 +1271,6 @@ static int ring_waves(int rtiles, int D) {
   return 8;
 }
 
-// Token-range split: enough (pair, row group, chunk) work items for about four rounds of
-// resident workgroups (1 per CU at 8 waves, 2 at 4, 4 at 1-2 waves: the LDS stage
-// buffers), chunks of at least 256 tokens, a whole number of stages each.
 struct AttnSplit { int nchunk, tpc, rows_pad, ngroups; };
 // compute units of the current device (256 on MI355X), queried once per device
 static int device_cus() {
@@ -1273,6 +1283,35 @@ static int device_cus() {
     cached[dev] = n;
   }
   return cached[dev];
+}
+
+// Token chunks per pair of the ring path: the count with the least estimated time, from
+//   rounds of resident workgroups x (a chunk's tokens + set-up)
+//     + writing the chunks' partial results and merging them (4 TB/s, and a launch).
+// Chunks hold at least 256 tokens.  Per-token times are a workgroup's, measured at the residency
+// that the LDS stages and registers allow (one workgroup per CU at 8 waves and at 4 of head dim
+// 256, else two).  Past three rounds the launch levels out and half a round is added instead of
+// rounding up.  Against four rounds of workgroups whatever the shape, as before: 2048 causal
+// queries over 6144 and 5003 tokens 677 -> 499 us (one chunk instead of two: 134 MB of partial
+// results less, and the longest groups first), 1000 queries of a head-dim-64 model 568 -> 388,
+// 300 queries over 20000 tokens 236 -> 180 (6 chunks instead of 26), 16 over 4 x 8k, 8 layers,
+// 275 -> 240.
+static int ring_chunks(int64_t items, int64_t rows, int tiles, int D, int span, int cus) {
+  const int64_t slots = (int64_t)cus * (tiles >= 8 || (D == 256 && tiles >= 4) ? 1 : 2);
+  const double us_token = D == 256 ? (tiles >= 4 ? 0.110 : 0.045) : D == 128 ? 0.048 : 0.038;
+  const double us_setup = 4.0, us_merge = 4.0, us_per_row_chunk = 2.0 * (D + 2) * sizeof(float) / 4.0e6;
+  const int most = std::max(1, span / 256);
+  int best = 1;
+  double best_us = 0.0;
+  for (int c = 1; c <= most; ++c) {
+    const double x = (double)items * c / (double)slots;
+    const double rounds = x <= 3.0 ? std::ceil(x) : x + 0.5;
+    double us = rounds * ((double)span / c * us_token + us_setup);
+    if (c > 1) us += us_merge + (double)rows * c * us_per_row_chunk;
+    if (c == 1 || us < best_us) { best_us = us; best = c; }
+    if (x > 8.0) break;   // more chunks only add set-ups and partial results
+  }
+  return best;
 }
 
 static AttnSplit attn_split(int pairs, int N, int G, int D, int span, int cus) {
@@ -1300,10 +1339,7 @@ static AttnSplit attn_split(int pairs, int N, int G, int D, int span, int cus) {
   const int st = ring_stage(tiles, D);
   sp.ngroups = (rtiles + tiles - 1) / tiles;
   sp.rows_pad = N * G;   // only rows that exist are written and merged
-  const int per_cu = tiles >= 8 || D == 256 ? 1 : 2;  // resident ring workgroups per CU (LDS)
-  const int64_t items = (int64_t)pairs * sp.ngroups;
-  const int64_t want = 4LL * 256 * per_cu;
-  int nchunk = (int)std::min<int64_t>(std::max<int64_t>(1, (want + items - 1) / items), std::max(1, span / 256));
+  const int nchunk = ring_chunks((int64_t)pairs * sp.ngroups, (int64_t)pairs * sp.rows_pad, tiles, D, span, cus);
   int tpc = ((span + nchunk - 1) / nchunk + st - 1) / st * st;
   tpc = std::max(tpc, st);
   sp.nchunk = (span + tpc - 1) / tpc;
@@ -1485,7 +1521,8 @@ extern "C" int actkv_paged_attention(
                       kv_sl % 8 == 0 && kv_sv % 8 == 0 && kv_sb % 8 == 0 && kv_ss % 8 == 0 &&
                       kv_sh % 8 == 0 && o_sl % 4 == 0 && o_sr % 4 == 0 && o_sn % 4 == 0 && o_sh % 4 == 0;
   const bool mfma_ok = q_dtype == kv_dtype && (kv_dtype == ACTKV_BF16 || kv_dtype == ACTKV_F16) &&
-                       (D == 256 || D == 128 || D == 64) && G >= 1 && vec_ok && bs_shift >= 0;
+                       (D == 256 || D == 128 || D == 64) && G >= 1 && vec_ok && bs_shift >= 0 &&
+                       (int64_t)block_size * kv_ss <= 0x7fffffffLL;   // byte offsets in a block: 32 bits
   if (mfma_ok) {
     void *ws = workspace;
     const size_t wb = workspace_bytes;
