@@ -701,14 +701,17 @@ attn_ring_kernel(AttnArgs a, int pairs, int ngroups, int bs_shift) {
   const int bid = blockIdx.x;
   const int xcd = bid & 7, jj = bid >> 3;
   const int per_pair = ngroups * a.nchunk;
-  const int p = (jj / per_pair) * 8 + xcd;
+  const int seq = (jj / per_pair) * 8 + xcd;
   // causal: the last groups see the most tokens and go first, so that the launch ends on short ones
   const int gpos = (jj % per_pair) / a.nchunk, chunk = jj % a.nchunk;
   const int grp = CAUSAL ? ngroups - 1 - gpos : gpos;
-  if (p >= pairs) return;
-  const int h = p % a.Hkv;
-  const int r = (p / a.Hkv) % a.R;
-  const int l = p / (a.Hkv * a.R);
+  if (seq >= pairs) return;
+  const int h = seq % a.Hkv;
+  const int l = seq / (a.Hkv * a.R);
+  // requests rotated by the layer: an XCD's workgroups go to its shader engines in turn, and with
+  // as many requests as engines the longest would always meet the same one
+  const int r = (seq / a.Hkv + l) % a.R;
+  const int p = (l * a.R + r) * a.Hkv + h;   // the pair, as the merge counts them
   const int nq = attn_nq(a, r);
   if (grp * NW * 32 >= nq * G) return;
   const int S_all = attn_seq_len(a, r);

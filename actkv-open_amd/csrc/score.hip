@@ -107,6 +107,58 @@ __device__ __forceinline__ int seq_len_of(const ScoreArgs &a, int r) {
   return s < 0 ? 0 : (s > span ? span : s);
 }
 
+// The (layer, request, head pack, token range) of position jj of an XCD's workgroup sequence.
+// An XCD's workgroups are dealt to its four shader engines in turn, whatever each still has to
+// do, so empty ranges (a request shorter than the longest, or without queries in this launch) and
+// long ones at regular positions leave engines idle.  With several requests the sequence
+// therefore holds only ranges with work: lane i of each wave counts request i's ranges, a scan
+// numbers them, and they are dealt out per (layer, head pack), each time rotated by one, every
+// request cut into equal ranges.  36 layers x 8 requests of 3300 to 14510 tokens with 64 to 250
+// queries: 3971 -> 3078 us; with up to 122 queries 2480 -> 1680, up to 60 1754 -> 1398, up to 30
+// 1440 -> 1203; head dim 256, 8 requests of 374 to 11244, 8 layers, 529 -> 375.  One request keeps the plain order (rotated, 36 x 32768 tokens took 1061 us against 1044).
+struct ScoreRange { int l, r, pack, t_begin, t_end; };
+template <int GRAN>
+__device__ __forceinline__ bool score_range(const ScoreArgs &a, int xcd, int jj, int pairs, int cpp, int tpw, int packs,
+                                            ScoreRange &o) {
+  if (a.R > 1 && a.R <= 64) {
+    const int lane = threadIdx.x & 63;
+    int S_l = 0, c_l = 0;
+    if (lane < a.R) {
+      S_l = seq_len_of(a, lane);
+      const int nq = a.n_valid ? min(max(a.n_valid[lane], 0), a.N) : a.N;
+      c_l = nq > a.qc0 ? (S_l + tpw - 1) / tpw : 0;
+    }
+    const int inc = (int)wave_scan_u32((uint32_t)c_l, 0u, OpAdd());
+    const int C = __builtin_amdgcn_readlane(inc, 63);
+    if (C == 0) return false;
+    // head packs that divide over the XCDs stay on theirs; others are dealt over all XCDs
+    const int hx = packs % 8 == 0 ? packs / 8 : packs;
+    const int seq = packs % 8 == 0 ? jj : jj * 8 + xcd;
+    const int unit = seq / C, e = (seq % C + unit) % C;
+    o.l = unit / hx;
+    o.pack = packs % 8 == 0 ? (unit % hx) * 8 + xcd : unit % hx;
+    if (o.l >= a.L) return false;
+    o.r = __builtin_ctzll(__builtin_amdgcn_ballot_w64(inc > e));
+    const int c = __builtin_amdgcn_readlane(c_l, o.r);
+    const int S = __builtin_amdgcn_readlane(S_l, o.r);
+    const int chunk = e - (__builtin_amdgcn_readlane(inc, o.r) - c);
+    const int per = ((S + c - 1) / c + GRAN - 1) / GRAN * GRAN;   // <= tpw, a multiple of GRAN
+    o.t_begin = chunk * per;
+    o.t_end = min(o.t_begin + per, S);
+    return o.t_begin < S;
+  }
+  const int p = (jj / cpp) * 8 + xcd;
+  const int chunk = a.R > 1 ? (jj + jj / cpp) % cpp : jj % cpp;
+  if (p >= pairs) return false;
+  o.pack = p % packs;
+  o.r = (p / packs) % a.R;
+  o.l = p / (packs * a.R);
+  const int S = seq_len_of(a, o.r);
+  o.t_begin = chunk * tpw;
+  o.t_end = min(o.t_begin + tpw, S);
+  return o.t_begin < S;
+}
+
 // ------------------------------------------------------------------ generic
 // grid (ceil(span/256), L*R*Hkv), 256 threads; one thread per token slot.
 template <typename QT, typename KT>
@@ -358,16 +410,9 @@ score_kslice_kernel(ScoreArgs a, int tpw, int cpp, int pairs, int bs_shift) {
   // from HBM into that XCD's L2 once.
   const int bid = blockIdx.x;
   const int xcd = bid & 7, jj = bid >> 3;
-  const int p = (jj / cpp) * 8 + xcd;
-  const int chunk = jj % cpp;
-  if (p >= pairs) return;
-  const int h = p % a.Hkv;
-  const int r = (p / a.Hkv) % a.R;
-  const int l = p / (a.Hkv * a.R);
-  const int S = seq_len_of(a, r);
-  const int t_begin = chunk * tpw;
-  if (t_begin >= S) return;
-  const int t_end = min(t_begin + tpw, S);
+  ScoreRange wr;
+  if (!score_range<32>(a, xcd, jj, pairs, cpp, tpw, a.Hkv, wr)) return;
+  const int h = wr.pack, r = wr.r, l = wr.l, t_begin = wr.t_begin, t_end = wr.t_end;
   const int nq_all = a.n_valid ? min(max(a.n_valid[r], 0), a.N) : a.N;
   const int nq = min(max(nq_all - a.qc0, 0), a.qcn);
   if (nq <= 0) return;
@@ -666,29 +711,12 @@ score_qreg_kernel(ScoreArgs a, int tpw, int cpp, int pairs, int bs_shift) {
 
   // XCD-aware work mapping: all token ranges of one (layer, request, head pack)
   // land on the same XCD (blockIdx % 8), so its query tiles are fetched from HBM
-  // into that XCD's L2 once.  With several requests the grid is sized for the
-  // longest, so the ranges past a shorter request's end are empty and its last one
-  // partial; each pair then takes its ranges in an order rotated by its place on
-  // the XCD, which spreads the empty and partial ones over the dispatch positions.
-  // In plain order range c always sits at position c mod 4 of the XCD's sequence,
-  // and with 8 ranges per pair the positions holding ranges 0 and 4 then carry
-  // most of the work (36 layers x 8 requests of 13103-58038 tokens: 9.29 ms plain,
-  // 8.65 ms rotated; uniform lengths in a table padded to 8 ranges: 10.9 ms plain,
-  // 9.0 ms rotated).  One request keeps the plain order (36 x 32768 tokens:
-  // 1.044 ms plain, 1.061 ms rotated).
+  // into that XCD's L2 once.
   const int bid = blockIdx.x;
   const int xcd = bid & 7, jj = bid >> 3;
-  const int p = (jj / cpp) * 8 + xcd;
-  const int chunk = a.R > 1 ? (jj + jj / cpp) % cpp : jj % cpp;
-  if (p >= pairs) return;
-  const int hpk = a.Hkv / HP;           // head packs per (layer, request)
-  const int h0 = (p % hpk) * HP;
-  const int r = (p / hpk) % a.R;
-  const int l = p / (hpk * a.R);
-  const int S = seq_len_of(a, r);
-  const int t_begin = chunk * tpw;
-  if (t_begin >= S) return;
-  const int t_end = min(t_begin + tpw, S);
+  ScoreRange wr;
+  if (!score_range<CH>(a, xcd, jj, pairs, cpp, tpw, a.Hkv / HP, wr)) return;
+  const int h0 = wr.pack * HP, r = wr.r, l = wr.l, t_begin = wr.t_begin, t_end = wr.t_end;
   const int nq_all = a.n_valid ? min(max(a.n_valid[r], 0), a.N) : a.N;
   const int nq = min(max(nq_all - a.qc0, 0), a.qcn);
   if (nq <= 0) return;
@@ -1127,10 +1155,13 @@ static int launch_mfma(const ScoreArgs &a0, int bs_shift, hipStream_t st) {
     // 3.5-4.4) and above 384 (the matrix cores bound it); the K-slice kernel from 129 to
     // 384 rows (with 2 heads per workgroup, 4 row groups each, or 1 head and 4 row
     // groups, the query-register kernel took 4-10% longer there)
+    // Above 384 rows with a query count per request the K-slice kernel again: its time follows
+    // each request's own row count, where the other's waves idle (8 requests of 55 to 122 of 122
+    // queries, 36 layers: 1928 against 1651 us; full tiles, 36 x 32k: 1091 against 1139).
     // groups of 8 and 16 heads, and groups padded to 4, 8 or 16 (3, 5-7, 9-15), run on the
     // query-register kernel alone (one head per workgroup)
     const bool qreg = DH != 128 || G >= 8 || a0.G != G || choice == MFMA_QREG ||
-                      (choice == MFMA_AUTO && (rows <= 128 || rows > 384));
+                      (choice == MFMA_AUTO && (rows <= 128 || (rows > 384 && !a0.n_valid)));
     if (qreg) {
       // query tile in registers, K shared through LDS; RG row groups of 64 rows over HPV
       // heads per workgroup, chunks of CHV tokens, the first one's set-up costing about
@@ -1300,12 +1331,11 @@ extern "C" int actkv_action_scores(
   int bs_shift = -1;
   for (int sh = 4; sh < 31; ++sh)
     if (block_size == (1 << sh)) bs_shift = sh;
-  // At head dim 256 up to 16 query rows stay on the float32 kernel, whose small workgroups reach
+  // At head dim 256 up to 8 query rows stay on the float32 kernel, whose small workgroups reach
   // the HBM rate and level out over ragged lengths (8 requests of 374 to 11244 tokens, 8 layers:
-  // 247 us with 2 rows, 376 with 16, against 529 on the matrix cores whatever the rows; 594
-  // against 533 with 32).
+  // 260 us with 2 rows, 277 with 8, 376 with 16; the matrix-core kernel 375 us whatever the rows).
   const bool mfma_ok = q_dtype == kv_dtype && (kv_dtype == ACTKV_BF16 || kv_dtype == ACTKV_F16) &&
-                       ((D == 256 && (int64_t)N * G > 16) || D == 128 || D == 64) && G >= 1 && G <= 16 &&
+                       ((D == 256 && (int64_t)N * G > 8) || D == 128 || D == 64) && G >= 1 && G <= 16 &&
                        scale > 0.f && vec_ok && bs_shift >= 0;
   int rc;
   if (mfma_ok) {
