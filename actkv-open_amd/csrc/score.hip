@@ -115,7 +115,8 @@ __device__ __forceinline__ int seq_len_of(const ScoreArgs &a, int r) {
 // numbers them, and they are dealt out per (layer, head pack), each time rotated by one, every
 // request cut into equal ranges.  36 layers x 8 requests of 3300 to 14510 tokens with 64 to 250
 // queries: 3971 -> 3078 us; with up to 122 queries 2480 -> 1680, up to 60 1754 -> 1398, up to 30
-// 1440 -> 1203; head dim 256, 8 requests of 374 to 11244, 8 layers, 529 -> 375.  One request keeps the plain order (rotated, 36 x 32768 tokens took 1061 us against 1044).
+// 1440 -> 1203; head dim 256, 8 requests of 374 to 11244, 8 layers, 529 -> 375.  One
+// request keeps the plain order (rotated, 36 x 32768 tokens took 1061 us against 1044).
 struct ScoreRange { int l, r, pack, t_begin, t_end; };
 template <int GRAN>
 __device__ __forceinline__ bool score_range(const ScoreArgs &a, int xcd, int jj, int pairs, int cpp, int tpw, int packs,
@@ -1334,8 +1335,12 @@ extern "C" int actkv_action_scores(
   // At head dim 256 up to 8 query rows stay on the float32 kernel, whose small workgroups reach
   // the HBM rate and level out over ragged lengths (8 requests of 374 to 11244 tokens, 8 layers:
   // 260 us with 2 rows, 277 with 8, 376 with 16; the matrix-core kernel 375 us whatever the rows).
+  // So do up to 16 rows of a small call, where its set-up is not repaid (10 rows over 18115 tokens
+  // 4 us less; 16 rows over one 32k-token layer 70 us against 58).
+  const bool few_rows = (int64_t)N * G <= 8 ||
+                        ((int64_t)N * G <= 16 && (int64_t)L * R * max_blocks * block_size <= 24576);
   const bool mfma_ok = q_dtype == kv_dtype && (kv_dtype == ACTKV_BF16 || kv_dtype == ACTKV_F16) &&
-                       ((D == 256 && (int64_t)N * G > 8) || D == 128 || D == 64) && G >= 1 && G <= 16 &&
+                       ((D == 256 && !few_rows) || D == 128 || D == 64) && G >= 1 && G <= 16 &&
                        scale > 0.f && vec_ok && bs_shift >= 0;
   int rc;
   if (mfma_ok) {
