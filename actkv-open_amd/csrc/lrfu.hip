@@ -129,6 +129,42 @@ __global__ void __launch_bounds__(256) lrfu_act_kernel(LrfuArgs a) {
   a.act[((int64_t)l * a.R + r) * a.act_sr + t] = lrfu_head_act(a, sbase, t, torch_body_end(S));
 }
 
+// The same for 8 heads in 16-byte aligned rows: four tokens per thread, one 16-byte load per head,
+// all eight in flight (4-byte loads left the reads at 2.4 TB/s).  grid (ceil(max_seq / 1024), L, R).
+// A quad lies wholly in or out of the torch body (torch_body_end is a multiple of 4).  The agent
+// loop's round, 36 layers x 4 requests of 15k to 18k tokens: 35.1 -> 27.7 us.
+__global__ void __launch_bounds__(256) lrfu_act8_kernel(LrfuArgs a) {
+  constexpr int HH = 8;
+  const int l = blockIdx.y, r = blockIdx.z;
+  const int S = min(max(a.seq_used[r], 0), a.max_seq);
+  const int P = a.prot ? min(max(a.prot[r], 0), S) : 0;
+  const int t = (P & ~3) + 4 * (int)(blockIdx.x * 256 + threadIdx.x);
+  if (t >= S) return;
+  const float *sbase = a.scores + (int64_t)l * a.s_sl + (int64_t)r * a.s_sr;
+  float *act = a.act + ((int64_t)l * a.R + r) * a.act_sr;
+  const int body_end = torch_body_end(S);
+  if (t + 4 > S) {                          // the last tokens one by one: no read past the row
+    for (int u = max(t, P); u < S; ++u) act[u] = lrfu_head_act(a, sbase, u, body_end);
+    return;
+  }
+  f32x4 hv[HH];
+#pragma unroll
+  for (int hh = 0; hh < HH; ++hh) hv[hh] = *(const f32x4 *)(sbase + t + (int64_t)hh * a.s_sh);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float v;
+    if (a.head_reduce == ACTKV_REDUCE_MAX) {
+      v = hv[0][j];
+#pragma unroll
+      for (int hh = 1; hh < HH; ++hh) v = nanmax(v, hv[hh][j]);
+    } else {
+      auto ld = [&](int hh) { return hv[hh][j]; };
+      v = __fdiv_rn(torch_sum(ld, HH, t < body_end), (float)HH);
+    }
+    if (t + j >= P) act[t + j] = v;
+  }
+}
+
 // grid (L, R), LT threads, after lrfu_act_kernel has written the action scores to the
 // workspace.  KMAX > 0: thread i keeps the action scores of its tokens t = P + i + j*LT
 // (j < KMAX, segments of up to KMAX*LT tokens) in registers, loaded once with all their
@@ -388,7 +424,10 @@ extern "C" int actkv_lrfu_update(const float *scores, int64_t s_sl, int64_t s_sr
   // tokens per segment past the protected prefix are at most max_seq
   const dim3 grid(L, R);
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(lrfu_act_kernel, dim3((max_seq + 255) / 256, L, R), dim3(256), 0, st, a);
+  if (H == 8 && ((uintptr_t)scores & 15u) == 0 && s_sl % 4 == 0 && s_sr % 4 == 0 && s_sh % 4 == 0)
+    hipLaunchKernelGGL(lrfu_act8_kernel, dim3((max_seq + 1023) / 1024, L, R), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL(lrfu_act_kernel, dim3((max_seq + 255) / 256, L, R), dim3(256), 0, st, a);
   int rc = actkv_check_launch();
   if (rc) return rc;
   if (max_seq <= 16 * LT) hipLaunchKernelGGL(lrfu_update_kernel<16>, grid, dim3(LT), 0, st, a);
