@@ -9,8 +9,9 @@
 // range's K rows from HBM exactly once.  Two MFMA kernels: above 384 query rows,
 // and up to 128, the tile sits in registers while K chunks are shared through LDS
 // (score_qreg_kernel: fewer LDS reads per MFMA; the matrix cores bound it above
-// 384 rows, HBM up to 128); from 129 to 384 rows each wave streams its own K
-// slices into registers against the tile in LDS (score_kslice_kernel).  Both compute
+// 384 rows, HBM up to 128); from 129 to 384 rows, and above where requests have their
+// own query counts, each wave streams its own K slices into registers against the tile
+// in LDS (score_kslice_kernel).  Both compute
 //
 //   acc[row, t] = q_row . k_t - lse_row / scale            (bf16/fp16 MFMA, fp32 acc)
 //   p[n, t]     = exp2(scale*log2(e) * max_g acc[(n,g), t]) (max over the GQA group
@@ -373,7 +374,8 @@ __global__ void __launch_bounds__(256) score_generic_rows_kernel(ScoreArgs a, in
 }
 
 // ------------------------------------------------------------------ MFMA, K slices in registers
-// For query tiles of at most 384 rows.  One workgroup (NW waves) owns a (layer, request, KV head) pair and a
+// For query tiles of 129 to 384 rows, and up to 512 where requests have their own query
+// counts.  One workgroup (NW waves) owns a (layer, request, KV head) pair and a
 // token range.  The pair's whole action-query tile -- rows (query n, group head g),
 // nq*G <= ROWS of them, head_dim 128, bf16/fp16 -- is staged ONCE into LDS
 // (rows padded to 272 bytes: conflict-free A-operand reads), with the
