@@ -1334,13 +1334,13 @@ extern "C" int actkv_action_scores(
   int bs_shift = -1;
   for (int sh = 4; sh < 31; ++sh)
     if (block_size == (1 << sh)) bs_shift = sh;
-  // At head dim 256 up to 8 query rows stay on the float32 kernel, whose small workgroups reach
-  // the HBM rate and level out over ragged lengths (8 requests of 374 to 11244 tokens, 8 layers:
-  // 260 us with 2 rows, 277 with 8, 376 with 16; the matrix-core kernel 375 us whatever the rows).
-  // So do up to 16 rows of a small call, where its set-up is not repaid (10 rows over 18115 tokens
-  // 4 us less; 16 rows over one 32k-token layer 70 us against 58).
-  const bool few_rows = (int64_t)N * G <= 8 ||
-                        ((int64_t)N * G <= 16 && (int64_t)L * R * max_blocks * block_size <= 24576);
+  // At head dim 256 up to 16 query rows stay on the float32 kernel, whose small workgroups reach
+  // the HBM rate and level out over ragged lengths: 8 requests of 374 to 11244 tokens, 8 layers,
+  // 260 us with 2 rows, 277 with 8, 376 with 16, where the matrix-core kernel takes 375 whatever
+  // the rows; one layer of 8 ragged requests with up to 8 queries, scored and evicted, 174 against
+  // 235.  (Of equal long requests it would gain from 12 rows on: 2 x 8k, 8 layers, 194 against
+  // 144.)  Above 16 rows the float32 kernel's time doubles.
+  const bool few_rows = (int64_t)N * G <= 16;
   const bool mfma_ok = q_dtype == kv_dtype && (kv_dtype == ACTKV_BF16 || kv_dtype == ACTKV_F16) &&
                        ((D == 256 && !few_rows) || D == 128 || D == 64) && G >= 1 && G <= 16 &&
                        scale > 0.f && vec_ok && bs_shift >= 0;

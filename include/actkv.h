@@ -78,7 +78,7 @@ const char *actkv_version(void);
  * bf16/fp16 q and K of one dtype with D = 256, 128 or 64 and Hq/Hkv from 1 to 16 run on the
  * matrix cores (groups of 3, 5-7 and 9-15 laid out as 4, 8 and 16 rows per query, the extra rows
  * padding; 512/G' queries per launch for the laid-out group G', 256/G' at D = 256, more
- * as several launches), at D = 256 above 8 query rows N*G (16 in a small call); every other
+ * as several launches), at D = 256 above 16 query rows N*G; every other
  * case uses float32 dot products.
  */
 int actkv_action_scores(
